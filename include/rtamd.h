@@ -209,7 +209,10 @@ int rt_closest_hit_stats(rt_ctx* ctx, const rt_scene* scene, const rt_ray* rays_
  * `tree`, which can change which of two hits at equal t is reported. */
 enum { RT_LAYOUT_AUTO = 0, RT_LAYOUT_F32 = 1, RT_LAYOUT_Q16 = 2, RT_LAYOUT_W4 = 3 };
 /* Tree of the packed traversal, read by rt_scene_upload:
- * RT_TREE_GIVEN   the caller's nodes (e.g. Bvh::createBvh's)
+ * RT_TREE_GIVEN   the caller's nodes (e.g. Bvh::createBvh's): they decide which
+ *                 of two hits at equal t is reported; the 4-wide layout walks
+ *                 a tree of its own over the same leaves where that is the
+ *                 better one
  * RT_TREE_DEVICE  a linear BVH built on the device at upload
  *                 (rt_bvh_build_device); the shader-order traversal keeps the
  *                 caller's nodes, and a scene given without nodes uses the

@@ -173,7 +173,7 @@ struct rt_batch {
     rt_ctx* ctx = nullptr;
     std::vector<rt_batch_item> items;
     uint32_t total = 0;
-    uint32_t stack_need = 0;           // 3 * max 4-wide height + 1
+    uint32_t stack_need = 0;           // most stack entries an item's scene needs, plus one
     uint64_t total_tris = 0;
     BatchEntry* d_table = nullptr;
     uint32_t* d_offsets = nullptr;
@@ -412,7 +412,7 @@ extern "C" int rt_batch_create(rt_ctx* ctx, const rt_batch_item* items, uint32_t
     rt_batch_config cfg = config ? *config : default_config();
     if (!valid_config(cfg)) return set_error(ctx, RT_ERR_INVALID, "rt_batch_create: invalid configuration");
     uint64_t total = 0;
-    uint32_t h4 = 0;
+    uint32_t need = 1;
     uint64_t tris = 0;
     for (uint32_t i = 0; i < n; ++i) {
         const rt_batch_item& it = items[i];
@@ -424,7 +424,7 @@ extern "C" int rt_batch_create(rt_ctx* ctx, const rt_batch_item* items, uint32_t
         if (it.count && (!it.rays_dev || !it.hits_dev || ((uintptr_t)it.rays_dev & 15u) || ((uintptr_t)it.hits_dev & 15u)))
             return set_error(ctx, RT_ERR_INVALID, "rt_batch_create: item " + std::to_string(i) + " buffers null or unaligned");
         total += it.count;
-        h4 = std::max(h4, it.scene->height4);
+        need = std::max(need, it.scene->stack4);
         tris += it.scene->info.num_triangles;
     }
     if (total > 0x7fffffffull) return set_error(ctx, RT_ERR_INVALID, "rt_batch_create: more than 2^31 rays");
@@ -433,7 +433,7 @@ extern "C" int rt_batch_create(rt_ctx* ctx, const rt_batch_item* items, uint32_t
     b->ctx = ctx;
     b->items.assign(items, items + n);
     b->total = (uint32_t)total;
-    b->stack_need = 3 * h4 + 1;
+    b->stack_need = need;
     b->total_tris = tris;
     b->cfg = cfg;
     int rc = RT_OK;

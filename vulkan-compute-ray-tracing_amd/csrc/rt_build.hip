@@ -171,26 +171,32 @@ __device__ inline int delta(const uint64_t* __restrict__ keys, int64_t n, int64_
     return 64 + __clz((int)((uint32_t)i ^ (uint32_t)j));
 }
 
+// Internal node i's range ends at i and j, and it splits after position g.
+__device__ inline void radix_split(const uint64_t* __restrict__ keys, int64_t N, int64_t i, int64_t& j, int64_t& g) {
+    const int d = delta(keys, N, i, i + 1) - delta(keys, N, i, i - 1) >= 0 ? 1 : -1;
+    const int dmin = delta(keys, N, i, i - d);
+    int64_t lmax = 2;
+    while (delta(keys, N, i, i + lmax * d) > dmin) lmax *= 2;
+    int64_t l = 0;
+    for (int64_t t = lmax / 2; t >= 1; t /= 2)
+        if (delta(keys, N, i, i + (l + t) * d) > dmin) l += t;
+    j = i + l * d;
+    const int dnode = delta(keys, N, i, j);
+    int64_t s = 0;
+    for (int64_t div = 2;; div *= 2) {
+        const int64_t t = (l + div - 1) / div;
+        if (delta(keys, N, i, i + (s + t) * d) > dnode) s += t;
+        if (t == 1) break;
+    }
+    g = i + s * d + (d < 0 ? -1 : 0);
+}
+
 __global__ __launch_bounds__(256) void k_radix_tree(const uint64_t* __restrict__ keys, uint32_t n,
                                                     rt_bvh_node* __restrict__ nodes, int32_t* __restrict__ far) {
     const int64_t N = n;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N - 1; i += (int64_t)gridDim.x * blockDim.x) {
-        const int d = delta(keys, N, i, i + 1) - delta(keys, N, i, i - 1) >= 0 ? 1 : -1;
-        const int dmin = delta(keys, N, i, i - d);
-        int64_t lmax = 2;
-        while (delta(keys, N, i, i + lmax * d) > dmin) lmax *= 2;
-        int64_t l = 0;
-        for (int64_t t = lmax / 2; t >= 1; t /= 2)
-            if (delta(keys, N, i, i + (l + t) * d) > dmin) l += t;
-        const int64_t j = i + l * d;
-        const int dnode = delta(keys, N, i, j);
-        int64_t s = 0;
-        for (int64_t div = 2;; div *= 2) {
-            const int64_t t = (l + div - 1) / div;
-            if (delta(keys, N, i, i + (s + t) * d) > dnode) s += t;
-            if (t == 1) break;
-        }
-        const int64_t g = i + s * d + (d < 0 ? -1 : 0);
+        int64_t j, g;
+        radix_split(keys, N, i, j, g);
         const int64_t lo = i < j ? i : j, hi = i < j ? j : i;
         const int32_t left = (int32_t)(lo == g ? (N - 1 + g) : g);
         const int32_t right = (int32_t)(hi == g + 1 ? (N - 1 + g + 1) : g + 1);
@@ -318,6 +324,8 @@ size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 }  // namespace
 }  // namespace rtamd
+
+#include "rt_wide.hpp"
 
 using namespace rtamd;
 

@@ -6,6 +6,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -120,7 +121,7 @@ struct PackedTree {
     std::vector<PNodeQ> qnodes;    // the same nodes, 16-bit fixed point
     std::vector<PNode4> w4nodes;   // the same tree, 4-wide
     int32_t root4 = kEmptyRoot;
-    uint32_t height4 = 0;          // 4-wide node depth
+    uint32_t stack4 = 0;           // stack entries a 4-wide traversal can hold, plus one
     QFrame frame{};
     int32_t root = kEmptyRoot;
     uint32_t height = 0;           // packed internal-node depth (stack bound)
@@ -139,6 +140,22 @@ SceneCheck check_scene(const rt_scene_desc& d);
 void pack_tree(const rt_scene_desc& d, PackedTree& out);
 void quantize_nodes(PackedTree& out);
 void widen_nodes(PackedTree& out);
+
+// The device-built 4-wide tree of an upload (rt_wide.hpp), between the build
+// that fixes its size and the emission into the scene's arrays.
+struct WideTree;
+struct WideTreeDelete { void operator()(WideTree* t) const; };
+constexpr uint32_t kMaxWideStack = 96;     // deepest stack a kernel variant holds
+// Builds it over `packed`'s leaves on stream s.  `out` stays null (and the
+// call succeeds) where the caller's tree is traversed as it is: fewer than
+// two triangles, no room for the scratch, or a caller's tree whose boxes sum
+// to less area.  `records` and `need` (stack entries, plus one) are set
+// beside `out`.  Waits for the build.
+int wide_build(rt_ctx* ctx, const PackedTree& packed, hipStream_t s, std::unique_ptr<WideTree, WideTreeDelete>& out,
+               uint32_t& records, uint32_t& need);
+// Writes the caller's records (nodes[0..), leaf refs moved), the device
+// tree's after them (its root first), and the triangles and their ids in its order.
+int wide_emit(rt_ctx* ctx, const WideTree& t, uint32_t records, PNode4* nodes, PTri* tris, int32_t* ids, hipStream_t s);
 
 }  // namespace rtamd
 
@@ -170,12 +187,16 @@ struct PreparedScene {
     bool sphere_tree = false;
     std::vector<SphereNode> snodes;
     bool with_pnodes = false, with_qnodes = false;   // binary records uploaded now
+    std::unique_ptr<WideTree, WideTreeDelete> wide;  // the tree the 4-wide traversal walks, or null: the caller's
+    uint32_t wide_records = 0, wide_need = 0;
     uint64_t bytes = 0;                 // device bytes scene_commit allocates
 };
 int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& out);
 int scene_commit(rt_ctx* ctx, PreparedScene& prep, rt_scene** out);
-// Device bytes of the 4-wide records and packed triangles as uploaded.
-uint64_t packed_record_bytes(const PackedTree& p);
+// Gives the prepared device tree and its scratch back; P.bytes follows.
+void scene_drop_wide(PreparedScene& P);
+// Device bytes of the 4-wide records (the device tree's `wide` among them) and packed triangles as uploaded.
+uint64_t packed_record_bytes(const PackedTree& p, uint32_t wide);
 // The binary node records of `layout` (RT_LAYOUT_F32 / RT_LAYOUT_Q16) for a
 // scene uploaded without them: rebuilt from the scene's device arrays.
 int scene_binary_records(rt_ctx* ctx, rt_scene* s, uint32_t layout);
@@ -193,8 +214,12 @@ struct rt_scene {
     rtamd::PNodeQ* d_qnodes = nullptr;
     rtamd::PNode4* d_w4nodes = nullptr;
     rtamd::QFrame frame{};
+    // d_w4nodes holds the caller's records from index 0 (its root first) and,
+    // from root4 on, the device-built tree's (wide); without one root4 is the
+    // caller's root.  Both trees' leaves name d_ptris slots.
     int32_t root4 = rtamd::kEmptyRoot;
-    uint32_t height4 = 0;
+    bool wide = false;
+    uint32_t stack4 = 0;              // stack entries either tree needs, plus one
     rtamd::PTri* d_ptris = nullptr;
     // d_w4nodes and d_ptris share one allocation when both fit in 4 GiB:
     // d_ptris = d_w4nodes + tri_off bytes, so a kernel addresses either
@@ -324,7 +349,7 @@ int launch_sphere_pass(rt_ctx* ctx, const TraceArgs& a, hipStream_t s);
 int launch_fill_u32(rt_ctx* ctx, uint32_t* p, uint32_t value, uint32_t count, hipStream_t s);
 
 // Batched traversal from caller-filled device tables (rt_batch.hip): the
-// server's per-slot launches.  stack_need = 3 * max 4-wide height + 1;
+// server's per-slot launches.  stack_need = the scenes' largest stack4;
 // `cursor` holds kCursorBlock words (reset by the launch).
 int launch_batch_dynamic(rt_ctx* ctx, const BatchIo& bio, uint32_t* cursor, uint32_t total, uint32_t stack_need,
                          uint32_t refill, hipStream_t s);

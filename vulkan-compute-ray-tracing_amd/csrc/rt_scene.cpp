@@ -199,7 +199,7 @@ void pack_tree(const rt_scene_desc& d, PackedTree& out) {
 void widen_nodes(PackedTree& out) {
     out.w4nodes.clear();
     out.w4nodes.reserve(out.nodes.size() / 2 + 1);
-    out.height4 = 0;
+    out.stack4 = 1;
     if (out.root == kEmptyRoot || out.root < 0) { out.root4 = out.root; return; }
     // the binary record i holds its two children's boxes (q16) and refs;
     // the 4-wide record of i takes its grandchildren through internal
@@ -228,7 +228,8 @@ void widen_nodes(PackedTree& out) {
         }
         const int32_t me = (int32_t)out.w4nodes.size();
         out.w4nodes.push_back(PNode4{});
-        out.height4 = std::max(out.height4, f.depth);
+        // up to three deferred children per record on the path
+        out.stack4 = std::max(out.stack4, 3u * f.depth + 1u);
         PNode4& w = out.w4nodes[me];
         for (int k = 0; k < 4; ++k) {
             if (k < n) {
@@ -327,23 +328,68 @@ int upload_array(rt_ctx* ctx, T** dst, const T* src, uint32_t n, uint64_t& bytes
 // they fit in 4 GiB (nodes first, triangles from the next 256-byte boundary;
 // the traversal then addresses both by 32-bit offsets from one base), else
 // in two.
-int upload_records(rt_ctx* ctx, rt_scene* s, const PackedTree& packed, uint64_t& bytes) {
-    const size_t nb = (sizeof(PNode4) * packed.w4nodes.size() + 255) / 256 * 256;
-    const size_t tb = sizeof(PTri) * packed.tris.size();
-    if (nb + tb >= (1ull << 32) || !nb || !tb) {
-        int rc = upload_array(ctx, &s->d_w4nodes, packed.w4nodes.data(), (uint32_t)packed.w4nodes.size(), bytes);
-        if (!rc) rc = upload_array(ctx, &s->d_ptris, packed.tris.data(), (uint32_t)packed.tris.size(), bytes);
-        s->tri_off = kSeparateArrays;
+// The triangles' ids (d_ptri_id) go with them.
+int upload_records(rt_ctx* ctx, rt_scene* s, const PreparedScene& P, uint64_t& bytes) {
+    const PackedTree& packed = P.packed;
+    const size_t records = packed.w4nodes.size() + (P.wide ? P.wide_records : 0u);
+    const size_t nb = (sizeof(PNode4) * records + 255) / 256 * 256;
+    const size_t tb = sizeof(PTri) * packed.tris.size(), ib = sizeof(int32_t) * packed.tri_id.size();
+    if (!records || !tb) {                                   // a single triangle, or none
+        int rc = upload_array(ctx, &s->d_ptris, packed.tris.data(), (uint32_t)packed.tris.size(), bytes);
+        if (!rc) rc = upload_array(ctx, &s->d_ptri_id, packed.tri_id.data(), (uint32_t)packed.tri_id.size(), bytes);
         return rc;
     }
-    char* base = nullptr;
-    RT_HIP(ctx, hipMalloc((void**)&base, nb + tb));
-    s->d_w4nodes = reinterpret_cast<PNode4*>(base);          // owns the allocation
-    s->d_ptris = reinterpret_cast<PTri*>(base + nb);
-    s->tri_off = (uint32_t)nb;
-    RT_HIP(ctx, hipMemcpy(base, packed.w4nodes.data(), sizeof(PNode4) * packed.w4nodes.size(), hipMemcpyHostToDevice));
-    RT_HIP(ctx, hipMemcpy(base + nb, packed.tris.data(), tb, hipMemcpyHostToDevice));
-    bytes += nb + tb;
+    if (nb + tb >= (1ull << 32)) {
+        RT_HIP(ctx, hipMalloc((void**)&s->d_w4nodes, sizeof(PNode4) * records));
+        RT_HIP(ctx, hipMalloc((void**)&s->d_ptris, tb));
+        bytes += sizeof(PNode4) * records + tb;
+    } else {
+        char* base = nullptr;
+        RT_HIP(ctx, hipMalloc((void**)&base, nb + tb));
+        s->d_w4nodes = reinterpret_cast<PNode4*>(base);      // owns the allocation
+        s->d_ptris = reinterpret_cast<PTri*>(base + nb);
+        s->tri_off = (uint32_t)nb;
+        bytes += nb + tb;
+    }
+    RT_HIP(ctx, hipMalloc((void**)&s->d_ptri_id, ib));
+    bytes += ib;
+    if (P.wide) {
+        const int rc = wide_emit(ctx, *P.wide, P.wide_records, s->d_w4nodes, s->d_ptris, s->d_ptri_id, nullptr);
+        if (rc) return rc;
+        // any stream may trace the scene once the upload returns
+        RT_HIP(ctx, hipStreamSynchronize(nullptr));
+        return RT_OK;
+    }
+    RT_HIP(ctx, hipMemcpy(s->d_w4nodes, packed.w4nodes.data(), sizeof(PNode4) * packed.w4nodes.size(), hipMemcpyHostToDevice));
+    RT_HIP(ctx, hipMemcpy(s->d_ptris, packed.tris.data(), tb, hipMemcpyHostToDevice));
+    RT_HIP(ctx, hipMemcpy(s->d_ptri_id, packed.tri_id.data(), ib, hipMemcpyHostToDevice));
+    return RT_OK;
+}
+
+// Binary records name the packer's triangle slots; with a device tree the
+// scene's triangles lie in that tree's order, so the records' leaf refs move
+// (a triangle under two leaves has two equal slots: either will do).
+int place_binary_refs(rt_ctx* ctx, const rt_scene* s, uint32_t num_triangles, PackedTree& packed) {
+    if (!s->wide) return RT_OK;
+    const size_t n = packed.tri_id.size();
+    std::vector<int32_t> ids, place;
+    try {
+        ids.resize(n);
+        place.assign(num_triangles, 0);
+    } catch (const std::bad_alloc&) {
+        return set_error(ctx, RT_ERR_NOMEM, "binary node records: host copy");
+    }
+    RT_HIP(ctx, hipMemcpy(ids.data(), s->d_ptri_id, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+    for (size_t k = 0; k < n; ++k) place[ids[k]] = (int32_t)k;
+    auto moved = [&](int32_t ref) { return ref >= 0 ? ref : ~place[packed.tri_id[~ref]]; };
+    for (PNode& p : packed.nodes) {
+        p.d.x = moved(p.d.x);
+        p.d.y = moved(p.d.y);
+    }
+    for (PNodeQ& q : packed.qnodes) {
+        q.ref0 = moved(q.ref0);
+        q.ref1 = moved(q.ref1);
+    }
     return RT_OK;
 }
 
@@ -457,11 +503,20 @@ int device_tree(rt_ctx* ctx, const rt_triangle* tris, uint32_t n, std::vector<rt
 
 namespace rtamd {
 
-uint64_t packed_record_bytes(const PackedTree& p) {
-    const uint64_t nb = (sizeof(PNode4) * (uint64_t)p.w4nodes.size() + 255) / 256 * 256;
+uint64_t packed_record_bytes(const PackedTree& p, uint32_t wide) {
+    const uint64_t records = sizeof(PNode4) * ((uint64_t)p.w4nodes.size() + wide);
+    const uint64_t nb = (records + 255) / 256 * 256;
     const uint64_t tb = sizeof(PTri) * (uint64_t)p.tris.size();
-    if (nb + tb >= (1ull << 32) || !nb || !tb) return sizeof(PNode4) * (uint64_t)p.w4nodes.size() + tb;
+    if (nb + tb >= (1ull << 32) || !nb || !tb) return records + tb;
     return nb + tb;
+}
+
+void scene_drop_wide(PreparedScene& P) {
+    if (!P.wide) return;
+    P.bytes -= packed_record_bytes(P.packed, P.wide_records);
+    P.wide.reset();
+    P.wide_records = P.wide_need = 0;
+    P.bytes += packed_record_bytes(P.packed, 0);
 }
 
 int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& P) {
@@ -497,6 +552,11 @@ int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& P) {
         }
         if (P.packed.height > kMaxPackedHeight) P.fast = false;
     }
+    if (P.fast) {
+        RT_HIP(ctx, hipSetDevice(ctx->device));
+        const int rc = wide_build(ctx, P.packed, nullptr, P.wide, P.wide_records, P.wide_need);
+        if (rc) return rc;
+    }
     P.desc = user;
     if (user.num_spheres > kSphereLinear && user.num_spheres <= kMaxTreeSpheres) {
         try {
@@ -514,7 +574,7 @@ int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& P) {
                  sizeof(rt_sphere) * (uint64_t)user.num_spheres;
     if (P.sphere_tree) b += sizeof(SphereNode) * (uint64_t)P.snodes.size();
     if (P.fast) {
-        b += packed_record_bytes(P.packed) + sizeof(int32_t) * (uint64_t)P.packed.tri_id.size();
+        b += packed_record_bytes(P.packed, P.wide_records) + sizeof(int32_t) * (uint64_t)P.packed.tri_id.size();
         if (P.with_pnodes) b += sizeof(PNode) * (uint64_t)P.packed.nodes.size();
         if (P.with_qnodes) b += sizeof(PNodeQ) * (uint64_t)P.packed.qnodes.size();
     }
@@ -527,7 +587,7 @@ int scene_commit(rt_ctx* ctx, PreparedScene& P, rt_scene** out) {
     *out = nullptr;
     RT_HIP(ctx, hipSetDevice(ctx->device));
     const rt_scene_desc* desc = &P.desc;
-    const PackedTree& packed = P.packed;
+    PackedTree& packed = P.packed;
     const bool fast = P.fast;
     rt_scene* s = new rt_scene();
     s->ctx = ctx;
@@ -542,12 +602,13 @@ int scene_commit(rt_ctx* ctx, PreparedScene& P, rt_scene** out) {
         if (P.sphere_tree &&
             (rc = upload_array(ctx, &s->d_snodes, P.snodes.data(), (uint32_t)P.snodes.size(), bytes))) break;
         if (fast) {
+            s->wide = P.wide != nullptr;
+            if ((rc = upload_records(ctx, s, P, bytes))) break;
+            if ((P.with_pnodes || P.with_qnodes) && (rc = place_binary_refs(ctx, s, desc->num_triangles, packed))) break;
             if (P.with_pnodes &&
                 (rc = upload_array(ctx, &s->d_pnodes, packed.nodes.data(), (uint32_t)packed.nodes.size(), bytes))) break;
             if (P.with_qnodes &&
                 (rc = upload_array(ctx, &s->d_qnodes, packed.qnodes.data(), (uint32_t)packed.qnodes.size(), bytes))) break;
-            if ((rc = upload_records(ctx, s, packed, bytes))) break;
-            if ((rc = upload_array(ctx, &s->d_ptri_id, packed.tri_id.data(), (uint32_t)packed.tri_id.size(), bytes))) break;
         }
     } while (0);
     if (rc) {
@@ -556,8 +617,9 @@ int scene_commit(rt_ctx* ctx, PreparedScene& P, rt_scene** out) {
     }
     s->root_ref = fast ? packed.root : kEmptyRoot;
     s->frame = packed.frame;
-    s->root4 = fast ? packed.root4 : kEmptyRoot;
-    s->height4 = fast ? packed.height4 : 0;
+    s->root4 = !fast ? kEmptyRoot : s->wide ? (int32_t)packed.w4nodes.size() : packed.root4;
+    s->stack4 = fast ? std::max(packed.stack4, P.wide_need) : 0;
+    P.wide.reset();
     s->packed_height = fast ? packed.height : 0;
     s->ref_height = P.chk.height;
     s->fast = fast;
@@ -614,7 +676,9 @@ int scene_binary_records(rt_ctx* ctx, rt_scene* s, uint32_t layout) {
         return set_error(ctx, RT_ERR_NOMEM, std::string("binary node records: ") + e.what());
     }
     uint64_t bytes = 0;
-    int rc = want_f ? upload_array(ctx, &s->d_pnodes, packed.nodes.data(), (uint32_t)packed.nodes.size(), bytes)
+    int rc = place_binary_refs(ctx, s, nt, packed);
+    if (rc) return rc;
+    rc = want_f ? upload_array(ctx, &s->d_pnodes, packed.nodes.data(), (uint32_t)packed.nodes.size(), bytes)
                     : upload_array(ctx, &s->d_qnodes, packed.qnodes.data(), (uint32_t)packed.qnodes.size(), bytes);
     if (rc) return rc;
     s->info.device_bytes += bytes;

@@ -216,7 +216,7 @@ int launch_slot(rt_server* S, Slot& sl) {
             e.win0 = 0;
             sl.h_offsets[i] = off;
             off += r->n;
-            need = std::max(need, 3u * sc->height4 + 1u);
+            need = std::max(need, sc->stack4);
             if (sc->info.num_triangles >= (1u << 17)) long_rays += r->n;
         }
         sl.h_offsets[ni] = off;
@@ -449,7 +449,7 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
         if (rc) return fail(S, rc, std::string("rt_server_scene_add: ") + rt_last_error(S->ctx));
         if (!prep.fast) return fail(S, RT_ERR_UNSUPPORTED, "rt_server_scene_add: scene without the packed traversal");
     }
-    const uint64_t bytes = prep.bytes;
+    uint64_t bytes = prep.bytes;
     const uint64_t budget = S->cfg.hbm_budget;
     // the least recently used scene without queued or running work
     auto pick_victim = [&]() -> uint64_t {
@@ -492,6 +492,14 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
     for (;;) {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || (uint64_t)free_b >= bytes + margin) break;
+        // the traversal tree and its scratch go before any resident scene
+        if (prep.wide) {
+            scene_drop_wide(prep);
+            std::lock_guard<std::mutex> lk(S->mu);
+            S->resident -= bytes - prep.bytes;
+            bytes = prep.bytes;
+            continue;
+        }
         uint64_t v = 0;
         {
             std::lock_guard<std::mutex> lk(S->mu);

@@ -353,8 +353,7 @@ int launch_trace_packed(rt_ctx* ctx, const TraceArgs& a, hipStream_t s) {
     if (!sc->fast) return set_error(ctx, RT_ERR_UNSUPPORTED, "packed traversal needs a tree that encloses its triangles");
     const bool stats = (a.node_visits && a.tri_tests) || a.sums;
     if (resolved_layout(ctx) == RT_LAYOUT_W4) {
-        // up to three deferred children per 4-wide node on the path
-        const uint32_t need = 3u * sc->height4 + 1u;
+        const uint32_t need = sc->stack4;
         if (need <= 24) return launch_w4<24>(ctx, a, s, stats);
         if (need <= 36) return launch_w4<36>(ctx, a, s, stats);
         if (need <= 48) return launch_w4<48>(ctx, a, s, stats);

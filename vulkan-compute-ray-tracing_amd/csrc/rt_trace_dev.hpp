@@ -106,9 +106,11 @@ __device__ __forceinline__ float plane_bias(double bo, float inv) {
     return (float)(-(0x1p23 + bo) * (double)inv);
 }
 
-// triIntersect + hit_triangle's accept test on a packed triangle.
-__device__ __forceinline__ bool tri_test(const PTri& tr, const f3& o, const f3& d, float tmin, float tbest,
-                                         float& t, float& u, float& v) {
+// triIntersect on a packed triangle, with hit_triangle's tests except its
+// upper bound: the ray meets it past tmin (accepted if t is also below the
+// closest t so far).
+__device__ __forceinline__ bool tri_meets(const PTri& tr, const f3& o, const f3& d, float tmin, float& t, float& u,
+                                          float& v) {
     f3 v0{tr.a.x, tr.a.y, tr.a.z};
     f3 a{tr.a.w, tr.b.x, tr.b.y};
     f3 b{tr.b.z, tr.b.w, tr.c.x};
@@ -120,7 +122,7 @@ __device__ __forceinline__ bool tri_test(const PTri& tr, const f3& o, const f3& 
     v = dot(q, a) * idet;
     t = dot(n, p) * idet;
     bool inside = !(u < 0.0f || u > 1.0f || v < 0.0f || (u + v) > 1.0f);
-    return inside && t > tmin && t < tbest;
+    return inside && t > tmin;
 }
 
 // hit_sphere (ray-trace-compute.comp:175-203): returns the accepted root
@@ -281,16 +283,21 @@ __device__ __forceinline__ float shfl_f(float x, uint32_t src) {
 // once a wave's rays are used up, its idle lanes would wait for the
 // longest rays of the wave.  Instead each idle lane takes the bottom entry of
 // a busy lane's stack -- the subtree that lane would visit last -- and
-// traverses it for the ray's owner (a helper).  The ordered traversal's
-// visiting sequence is cut into pieces: a lane holds the piece
-// [plo, plo + 2^pk), and a steal halves the donor's piece, the donor keeping
-// the first half (its own remaining work) and the helper the second (the
-// stolen subtree, which comes after it).  Each piece accepts hits as the
-// whole traversal would (strictly closer than its best so far); a helper
-// starts from the donor's closest t, and at its end hands (t, piece, hit) to
-// the owner, who keeps the smaller t and on equal t the earlier piece.  The
-// result is the whole traversal's: the closest t, first in visiting order.
-// The owner writes it once its own piece and every helper have finished.
+// traverses it for the ray's owner (a helper).  A helper starts from the
+// donor's closest hit, and at its end hands its own to the owner, who keeps
+// the smaller t and writes it once its own part and every helper have
+// finished.
+//
+// Ties (4-wide layouts).  Of several hits at exactly equal t the caller's
+// tree names the one reported: the first in the order in which a traversal
+// of its records alone visits them.  This loop walks another tree
+// (rt_scene::root4) in shared pieces, so it only notes that its closest t
+// was met twice (`tie`); every box that holds a hit at the closest t is
+// visited, so no tie is missed.  A ray that ends with a tie is traced again
+// by one lane (`exact`) through the caller's records, whose root is record
+// 0, with its closest t as an inclusive bound: only boxes up to that t are
+// visited, in the order of a full traversal (a child's place among its
+// siblings depends on entry distances alone), and the first hit met is kept.
 template <int BLOCK, int STACK, int LAYOUT, bool STATS, bool BATCHED, int RING>
 __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const TraceIo& io, const BatchIo& bio,
                                                  int32_t* __restrict__ stk, int32_t* __restrict__ spill) {
@@ -354,13 +361,12 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
     uint64_t sum_nv = 0, sum_nt = 0;   // STATS: this lane's totals over its rays
     int sp = 0;
     int32_t cur = 0;
-    // work sharing (STEAL): the stack holds entries [bot, sp); the lane's
-    // piece of its ray's visiting sequence is [plo, plo + 2^pk)
+    bool tie = false;               // best_t was met by two triangles
+    bool exact = false;             // second trace of a tied ray, through the caller's records
+    // work sharing (STEAL): the stack holds entries [bot, sp)
     int bot = 0;
-    uint32_t plo = 0, pk = 31;
     int32_t owner = -1;             // a helper's owner lane; -1 for the owner
     uint32_t pending = 0;           // owner: helpers still running
-    uint32_t best_lo = 0;           // the piece that found `best`
     // owner whose own piece is done while helpers still run: not busy (it
     // takes no steps), not idle (it keeps its ray); only in a drained wave
     bool waiting = false;
@@ -481,13 +487,15 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                                           __uint_as_float(c.w))};
                 if (STATS) nt++;
                 float t, u, v;
-                // a best handed over from a later piece yields to an equal t of this one
-                float cap = best_t;
-                if (SH && best_lo > plo) cap = __uint_as_float(__float_as_uint(best_t) + 1u);
-                if (tri_test(tr, r.o, r.d, r.tmin, cap, t, u, v)) {
-                    best_t = t; bu = u; bv = v; best = slot;
-                    best_rel = t - t_shift;
-                    if (SH) best_lo = plo;
+                if (tri_meets(tr, r.o, r.d, r.tmin, t, u, v)) {
+                    const bool equal = t == best_t;
+                    if (t < best_t || (equal && exact && best < 0)) {
+                        best_t = t; bu = u; bv = v; best = slot;
+                        best_rel = t - t_shift;
+                        tie = false;
+                    } else if (equal && best >= 0) {
+                        tie = true;
+                    }
                 }
             }
         } else if (sp >= 0) {
@@ -529,7 +537,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                 PTri tr{tp[0], tp[1], tp[2]};
                 if (STATS) nt++;
                 float t, u, v;
-                if (tri_test(tr, r.o, r.d, r.tmin, best_t, t, u, v)) {
+                if (tri_meets(tr, r.o, r.d, r.tmin, t, u, v) && t < best_t) {
                     best_t = t; bu = u; bv = v; best = slot;
                     best_rel = t - t_shift;
                 }
@@ -539,11 +547,17 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
             if (sp > (SH ? bot : 0)) {
                 cur = pop();
             } else if (SH && owner >= 0) {
-                handoff = true;             // a helper's piece is done
+                handoff = true;             // a helper's part is done
                 busy = false;
             } else if (SH && pending != 0) {
-                waiting = true;             // the owner's piece is done
+                waiting = true;             // the owner's part is done
                 busy = false;
+            } else if (kW4 && tie && !exact) {
+                exact = true;               // best_t and best_rel stay as bounds
+                best = -1;
+                cur = 0;
+                sp = 0;
+                if (SH) bot = 0;
             } else {
                 // ---- ray finished: the result (spheres follow in their own pass)
                 const int32_t id = best >= 0 ? l_triid[best] : -1;
@@ -628,7 +642,8 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                     best_rel = r.tmax - t_shift;
                     best_t = r.tmax; bu = 0.0f; bv = 0.0f; best = -1;
                     nv = 0; nt = 0; sp = 0;
-                    bot = 0; plo = 0; pk = 31; owner = -1; pending = 0; best_lo = 0;
+                    tie = false; exact = false;
+                    bot = 0; owner = -1; pending = 0;
                     cur = root;
                     busy = true;
                     // an empty tree, or a ray that misses the frame's box
@@ -650,11 +665,12 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                 // would visit last, often culled by then).  Culling only: the
                 // closest hit and its ties lie at or before the owner's t, so
                 // no box that holds them is dropped, and acceptance still
-                // compares with the helper's own best.
+                // compares with the helper's own best.  A tied ray's second
+                // trace is never shared: its visiting order is the result.
                 const float owner_rel = shfl_f(best_rel, owner < 0 ? lane : (uint32_t)owner);
                 if (busy && owner >= 0) best_rel = fminf(best_rel, owner_rel);
                 const uint64_t idle_m = __ballot(!busy && !waiting);
-                const uint64_t donor_m = __ballot(busy && pk > 0 && sp - bot >= 1);
+                const uint64_t donor_m = __ballot(busy && !exact && sp - bot >= 1);
                 if ((uint32_t)__popcll(idle_m) >= io.steal && donor_m != 0) {
                     const uint32_t k = min((uint32_t)__popcll(idle_m), (uint32_t)__popcll(donor_m));
                     const uint32_t rank_idle = (uint32_t)__popcll(idle_m & lanes_below);
@@ -671,9 +687,10 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                     const float tsh = shfl_f(t_shift, src), tminr = shfl_f(tmin_rel, src);
                     const float bestr = shfl_f(best_rel, src), bestt = shfl_f(best_t, src);
                     const int v_bot = __shfl(bot, (int)src);
-                    const uint32_t v_plo = (uint32_t)__shfl((int)plo, (int)src);
-                    const uint32_t v_best_lo = (uint32_t)__shfl((int)best_lo, (int)src);
-                    const uint32_t v_pk = (uint32_t)__shfl((int)pk, (int)src);
+                    const float v_bu = shfl_f(bu, src), v_bv = shfl_f(bv, src);
+                    // its hit, and whether its t was met twice
+                    const int32_t v_best = __shfl(best, (int)src);
+                    const int v_tie = __shfl((int)tie, (int)src);
                     const int32_t v_owner = __shfl(owner < 0 ? (int32_t)lane : owner, (int)src);
                     // batched lanes each carry their item's scene
                     auto shfl_ptr = [&](const void* q) -> uint64_t {
@@ -706,23 +723,15 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                         tmin_rel = tminr;
                         best_rel = bestr;
                         best_t = bestt;
-                        bu = 0.0f; bv = 0.0f; best = -1;
+                        bu = v_bu; bv = v_bv; best = v_best;
+                        tie = v_tie != 0;
+                        exact = false;
                         sp = 0; bot = 0;
-                        pk = v_pk - 1u;
-                        plo = v_plo + (1u << pk);
-                        // the donor's best keeps the piece it came from: a
-                        // best an earlier helper handed over may come from a
-                        // piece after this one, and then an equal t found
-                        // here must replace it (the cap rule in step)
-                        best_lo = v_best_lo;
                         owner = v_owner;
                         pending = 0;
                         busy = true;
                     }
-                    if (donor) {
-                        bot++;
-                        pk--;
-                    }
+                    if (donor) bot++;
                     // owners count the helpers they gained
                     uint64_t tm = __ballot(thief);
                     while (tm != 0) {
@@ -751,12 +760,16 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                     const float ht = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(best_t), j));
                     const float hu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bu), j));
                     const float hv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bv), j));
-                    const uint32_t hlo = (uint32_t)__builtin_amdgcn_readlane((int)plo, j);
+                    const bool htie = __builtin_amdgcn_readlane((int)tie, j) != 0;
                     if ((int32_t)lane == o) {
                         pending--;
-                        if (hb >= 0 && (ht < best_t || (ht == best_t && hlo < best_lo))) {
-                            best = hb; best_t = ht; bu = hu; bv = hv; best_lo = hlo;
+                        // (a helper may bring back the hit it started from)
+                        if (hb >= 0 && ht < best_t) {
+                            best = hb; best_t = ht; bu = hu; bv = hv;
                             best_rel = ht - t_shift;
+                            tie = htie;
+                        } else if (hb >= 0 && ht == best_t) {
+                            tie = tie || htie || hb != best;
                         }
                     }
                 }
