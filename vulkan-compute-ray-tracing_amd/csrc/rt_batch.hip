@@ -209,7 +209,7 @@ int launch_batch_kernel(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
         if (per_cu < 1) per_cu = 1;
         if (b->cfg.blocks_per_cu && (int)b->cfg.blocks_per_cu < per_cu) per_cu = (int)b->cfg.blocks_per_cu;
         uint32_t blocks = (uint32_t)ctx->num_cus * (uint32_t)per_cu;
-        uint32_t need = (b->total + BLOCK - 1) / BLOCK;
+        uint32_t need = (b->total + BLOCK / 64 - 1) / (BLOCK / 64);
         b->grid_blocks = need < blocks ? need : blocks;
         size_t bytes = RING ? (size_t)(STACK - RING) * b->grid_blocks * BLOCK * sizeof(int32_t) : 0;
         if (bytes > b->spill_bytes) {
@@ -378,7 +378,7 @@ int launch_dyn_t(rt_ctx* ctx, const BatchIo& bio, uint32_t* cursor, uint32_t tot
     RT_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, 0));
     if (per_cu < 1) per_cu = 1;
     uint32_t blocks = (uint32_t)ctx->num_cus * (uint32_t)per_cu;
-    uint32_t need = (total + 255u) / 256u;
+    uint32_t need = (total + 3u) / 4u;
     if (need < blocks) blocks = need;
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, s, cursor, 0u, kCursorBlock);
     TraceIo io{nullptr, nullptr, nullptr, nullptr, nullptr, cursor, total, refill, nullptr,
