@@ -232,12 +232,13 @@ typedef struct rt_tuning {
                                traversals) 28 for queries and 24 for render
                                bounces, 48 below (short ones)                    */
     uint32_t blocks_per_cu; /* persistent blocks per CU (0 = occupancy limit)     */
-    uint32_t stack_lds;     /* 4-wide layout: 0 = whole traversal stack in LDS;
-                               8, 16 or 32 = that many top entries in LDS, deeper
-                               ones spill to HBM (more waves fit per CU)          */
+    uint32_t stack_lds;     /* 4-wide layout: 0 = the whole traversal stack in LDS
+                               where the launch's blocks fit a CU like that, else
+                               its first 24 entries; 8, 16 or 32 = that many
+                               entries in LDS; deeper ones spill to HBM          */
     uint32_t tree;          /* RT_TREE_*                                          */
     uint32_t ray_order;     /* RT_ORDER_*: the order a query's rays are traced in */
-    uint32_t steal;         /* 4-wide layout, whole stack in LDS: once a wave's
+    uint32_t steal;         /* 4-wide layout: once a wave's
                                rays are used up, this many idle lanes (1..64)
                                make it hand subtrees from its busy lanes' stacks
                                to the idle ones (hits unchanged); 0 = 32,
@@ -266,8 +267,8 @@ typedef struct rt_batch_item {
 
 typedef struct rt_batch_config {
     uint32_t block;          /* threads per work-group: 128 or 256 (0 = 256)       */
-    uint32_t stack_lds;      /* 0 = whole stack in LDS; 8, 16 or 32 = top entries
-                                (4-wide records only)                             */
+    uint32_t stack_lds;      /* 0 = the first 24 stack entries in LDS; 8, 16 or 32
+                                = that many (4-wide records only)                 */
     uint32_t regroup;        /* 0 = rays in the caller's order; 1 = bin each item's
                                 rays by origin cell (16^3, Morton order); 2 = by
                                 direction octant, then origin cell (8^3)          */

@@ -86,6 +86,8 @@ extern "C" int rt_destroy(rt_ctx* ctx) {
     (void)hipDeviceSynchronize();
     for (int i = 0; i < rt_ctx::kWorkspaces; ++i)
         if (ctx->ws[i]) (void)hipFree(ctx->ws[i]);
+    for (int32_t* p : ctx->d_spill)
+        if (p) (void)hipFree(p);
     if (ctx->d_counters) (void)hipFree(ctx->d_counters);
     if (ctx->d_cursors) (void)hipFree(ctx->d_cursors);
     if (ctx->d_render_sums) (void)hipFree(ctx->d_render_sums);

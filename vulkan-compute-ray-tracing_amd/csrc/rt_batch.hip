@@ -121,11 +121,11 @@ __global__ __launch_bounds__(256) void k_regroup_scatter(BatchIo bio, uint32_t t
     }
 }
 
-template <int BLOCK, int STACK, int RING, int LAYOUT>
+template <int BLOCK, int STACK, bool DEEP, int LAYOUT>
 __global__ __launch_bounds__(BLOCK) void k_trace_batch(TraceIo io, BatchIo bio, int32_t* spill) {
-    __shared__ int32_t stk[(RING ? RING : STACK) * BLOCK];
+    __shared__ int32_t stk[STACK * BLOCK];
     TraceScene sc{};
-    trace_persistent<BLOCK, STACK, LAYOUT, false, true, RING>(sc, io, bio, stk, spill);
+    trace_persistent<BLOCK, STACK, LAYOUT, false, true, DEEP>(sc, io, bio, stk, spill);
 }
 
 __global__ void k_fill(uint32_t* p, uint32_t value, uint32_t count) {
@@ -199,9 +199,9 @@ struct rt_batch {
 
 namespace {
 
-template <int BLOCK, int STACK, int RING, int LAYOUT>
+template <int BLOCK, int STACK, bool DEEP, int LAYOUT>
 int launch_batch_kernel(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
-    auto kern = k_trace_batch<BLOCK, STACK, RING, LAYOUT>;
+    auto kern = k_trace_batch<BLOCK, STACK, DEEP, LAYOUT>;
     if (b->dry) {
         // occupancy and the spill buffer are settled outside any capture
         int per_cu = 0;
@@ -209,9 +209,8 @@ int launch_batch_kernel(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
         if (per_cu < 1) per_cu = 1;
         if (b->cfg.blocks_per_cu && (int)b->cfg.blocks_per_cu < per_cu) per_cu = (int)b->cfg.blocks_per_cu;
         uint32_t blocks = (uint32_t)ctx->num_cus * (uint32_t)per_cu;
-        uint32_t need = (b->total + BLOCK / 64 - 1) / (BLOCK / 64);
-        b->grid_blocks = need < blocks ? need : blocks;
-        size_t bytes = RING ? (size_t)(STACK - RING) * b->grid_blocks * BLOCK * sizeof(int32_t) : 0;
+        b->grid_blocks = plan_launch(b->total, blocks, BLOCK / 64, device_simds(ctx)).blocks;
+        size_t bytes = DEEP ? (size_t)(b->stack_need - STACK) * b->grid_blocks * BLOCK * sizeof(int32_t) : 0;
         if (bytes > b->spill_bytes) {
             RT_HIP(ctx, hipDeviceSynchronize());
             if (b->d_spill) RT_HIP(ctx, hipFree(b->d_spill));
@@ -223,44 +222,37 @@ int launch_batch_kernel(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
     }
     const uint32_t blocks = b->grid_blocks;
     if (!blocks) return RT_OK;
-    int32_t* spill = RING ? b->d_spill : nullptr;
+    int32_t* spill = DEEP ? b->d_spill : nullptr;
     TraceIo io{nullptr, nullptr, nullptr, nullptr, nullptr, b->d_cursor, b->total, b->cfg.refill, nullptr,
-               b->total >= (1u << 16) ? kSegments : 1u, drain_steal(ctx)};
+               b->total >= (1u << 16) ? kSegments : 1u, drain_steal(ctx), device_simds(ctx)};
     BatchIo bio{b->d_table, b->d_offsets, b->d_chunk_item, b->cfg.regroup ? b->d_perm : nullptr};
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(BLOCK), 0, s, io, bio, spill);
     RT_HIP(ctx, hipGetLastError());
     return RT_OK;
 }
 
-template <int BLOCK, int STACK>
-int launch_batch_ring(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
-    if (b->cfg.stack_lds == 8 && STACK > 8) return launch_batch_kernel<BLOCK, STACK, 8, kLayoutW4>(ctx, b, s);
-    if (b->cfg.stack_lds == 16 && STACK > 16) return launch_batch_kernel<BLOCK, STACK, 16, kLayoutW4>(ctx, b, s);
-    if (b->cfg.stack_lds == 32 && STACK > 32) return launch_batch_kernel<BLOCK, STACK, 32, kLayoutW4>(ctx, b, s);
-    return launch_batch_kernel<BLOCK, STACK, 0, kLayoutW4>(ctx, b, s);
-}
-
 // Binary 16-bit records: one deferred child per level, whole stack in LDS.
 template <int BLOCK>
 int launch_batch_binary(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
     const uint32_t h = b->packed_height;
-    if (h <= 24) return launch_batch_kernel<BLOCK, 24, 0, kLayoutQ16>(ctx, b, s);
-    if (h <= 32) return launch_batch_kernel<BLOCK, 32, 0, kLayoutQ16>(ctx, b, s);
-    if (h <= 48) return launch_batch_kernel<BLOCK, 48, 0, kLayoutQ16>(ctx, b, s);
-    if (h <= 64) return launch_batch_kernel<BLOCK, 64, 0, kLayoutQ16>(ctx, b, s);
+    if (h <= 24) return launch_batch_kernel<BLOCK, 24, false, kLayoutQ16>(ctx, b, s);
+    if (h <= 32) return launch_batch_kernel<BLOCK, 32, false, kLayoutQ16>(ctx, b, s);
+    if (h <= 48) return launch_batch_kernel<BLOCK, 48, false, kLayoutQ16>(ctx, b, s);
+    if (h <= 64) return launch_batch_kernel<BLOCK, 64, false, kLayoutQ16>(ctx, b, s);
     return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: a binary tree deeper than 64 levels");
 }
 
 template <int BLOCK>
 int launch_batch_block(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
     if (binary_layout(b->cfg)) return launch_batch_binary<BLOCK>(ctx, b, s);
+    // the first entries of each lane's stack in LDS, the rest in b->d_spill
     const uint32_t need = b->stack_need;
-    if (need <= 24) return launch_batch_ring<BLOCK, 24>(ctx, b, s);
-    if (need <= 36) return launch_batch_ring<BLOCK, 36>(ctx, b, s);
-    if (need <= 48) return launch_batch_ring<BLOCK, 48>(ctx, b, s);
-    if (need <= 64) return launch_batch_ring<BLOCK, 64>(ctx, b, s);
-    if (need <= 96) return launch_batch_ring<BLOCK, 96>(ctx, b, s);
-    return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: a 4-wide tree deeper than 31 levels");
+    if (need > kMaxWideStack) return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: a 4-wide tree deeper than 31 levels");
+    if (need <= kStackLds) return launch_batch_kernel<BLOCK, kStackLds, false, kLayoutW4>(ctx, b, s);
+    if (b->cfg.stack_lds == 8) return launch_batch_kernel<BLOCK, 8, true, kLayoutW4>(ctx, b, s);
+    if (b->cfg.stack_lds == 16) return launch_batch_kernel<BLOCK, 16, true, kLayoutW4>(ctx, b, s);
+    if (b->cfg.stack_lds == 32) return launch_batch_kernel<BLOCK, 32, true, kLayoutW4>(ctx, b, s);
+    return launch_batch_kernel<BLOCK, kStackLds, true, kLayoutW4>(ctx, b, s);
 }
 
 // The whole launch sequence on `s` (also what the graph captures).
@@ -371,19 +363,25 @@ std::string cache_key(const rt_batch* b) {
     return k.str();
 }
 
-template <int STACK>
-int launch_dyn_t(rt_ctx* ctx, const BatchIo& bio, uint32_t* cursor, uint32_t total, uint32_t refill, hipStream_t s) {
-    auto kern = k_trace_batch<256, STACK, 0, kLayoutW4>;
+template <bool DEEP>
+int launch_dyn_t(rt_ctx* ctx, const BatchIo& bio, uint32_t* cursor, uint32_t total, uint32_t stack_need,
+                 uint32_t refill, hipStream_t s) {
+    auto kern = k_trace_batch<256, kStackLds, DEEP, kLayoutW4>;
+    int32_t* spill = nullptr;
+    if (DEEP) {
+        const int rc = stack_spill(ctx, stack_need - kStackLds, s, &spill);
+        if (rc) return rc;
+        if (!spill) return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: no stack spill area");
+    }
     int per_cu = 0;
     RT_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, 0));
     if (per_cu < 1) per_cu = 1;
     uint32_t blocks = (uint32_t)ctx->num_cus * (uint32_t)per_cu;
-    uint32_t need = (total + 3u) / 4u;
-    if (need < blocks) blocks = need;
+    blocks = plan_launch(total, blocks, 4u, device_simds(ctx)).blocks;
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, s, cursor, 0u, kCursorBlock);
     TraceIo io{nullptr, nullptr, nullptr, nullptr, nullptr, cursor, total, refill, nullptr,
-               total >= (1u << 16) ? kSegments : 1u, drain_steal(ctx)};
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, s, io, bio, (int32_t*)nullptr);
+               total >= (1u << 16) ? kSegments : 1u, drain_steal(ctx), device_simds(ctx)};
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, s, io, bio, spill);
     RT_HIP(ctx, hipGetLastError());
     return RT_OK;
 }
@@ -395,12 +393,9 @@ int launch_batch_dynamic(rt_ctx* ctx, const BatchIo& bio, uint32_t* cursor, uint
                          uint32_t refill, hipStream_t s) {
     if (!total) return RT_OK;
     if (refill < 1u || refill > 64u) refill = 32u;
-    if (stack_need <= 24) return launch_dyn_t<24>(ctx, bio, cursor, total, refill, s);
-    if (stack_need <= 36) return launch_dyn_t<36>(ctx, bio, cursor, total, refill, s);
-    if (stack_need <= 48) return launch_dyn_t<48>(ctx, bio, cursor, total, refill, s);
-    if (stack_need <= 64) return launch_dyn_t<64>(ctx, bio, cursor, total, refill, s);
-    if (stack_need <= 96) return launch_dyn_t<96>(ctx, bio, cursor, total, refill, s);
-    return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: a 4-wide tree deeper than 31 levels");
+    if (stack_need > kMaxWideStack) return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: a 4-wide tree deeper than 31 levels");
+    return stack_need <= kStackLds ? launch_dyn_t<false>(ctx, bio, cursor, total, stack_need, refill, s)
+                                   : launch_dyn_t<true>(ctx, bio, cursor, total, stack_need, refill, s);
 }
 }  // namespace rtamd
 

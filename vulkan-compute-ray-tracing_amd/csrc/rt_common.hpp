@@ -26,6 +26,8 @@ static_assert(sizeof(rt_sphere) == 32 && offsetof(rt_sphere, materialIndex) == 1
 static_assert(sizeof(rt_ubo) == 32 && offsetof(rt_ubo, currentSample) == 16, "UBO");
 static_assert(sizeof(rt_ray) == 32 && sizeof(rt_hit) == 16, "ray/hit");
 
+#define RT_HOST_DEVICE __host__ __device__
+
 namespace rtamd {
 
 // ---------------------------------------------------------------------------
@@ -145,7 +147,9 @@ void widen_nodes(PackedTree& out);
 // that fixes its size and the emission into the scene's arrays.
 struct WideTree;
 struct WideTreeDelete { void operator()(WideTree* t) const; };
-constexpr uint32_t kMaxWideStack = 96;     // deepest stack a kernel variant holds
+constexpr uint32_t kMaxWideStack = 96;     // deepest stack a traversal may need
+constexpr uint32_t kStackLds = 24;         // entries of a lane's stack in LDS, 4-wide layout
+constexpr uint32_t kMaxLanesPerCu = 2048;  // of any launch: 8 waves on each of 4 SIMDs
 // Builds it over `packed`'s leaves on stream s.  `out` stays null (and the
 // call succeeds) where the caller's tree is traversed as it is: fewer than
 // two triangles, no room for the scratch, or a caller's tree whose boxes sum
@@ -245,11 +249,12 @@ struct rt_ctx {
     std::string err;
     int num_cus = 0;
     // grow-only device workspaces: [0] render path state, [1] reference
-    // traversal stacks, [2] statistics scratch, [3] traversal stack spill,
-    // [4] BVH builder scratch, [5] ray-order keys and permutation
-    static constexpr int kWorkspaces = 6;
+    // traversal stacks, [2] statistics scratch, [3] BVH builder scratch,
+    // [4] ray-order keys and permutation
+    static constexpr int kWorkspaces = 5;
     void* ws[kWorkspaces] = {};
     size_t ws_bytes[kWorkspaces] = {};
+    int32_t* d_spill[3] = {};         // stack entries past LDS (stack_spill), each made on first use
     uint32_t* d_counters = nullptr;   // kRenderCounters words: a render's live rays per bounce
     uint32_t* d_cursors = nullptr;    // ring of persistent-kernel ray cursors
     uint32_t cursor_next = 0;
@@ -281,7 +286,7 @@ int set_error(rt_ctx* ctx, int code, const std::string& msg);
 // Triangles of one OBJ file (rt_obj.cpp); err receives the reason on failure.
 int obj_triangles(const char* path, uint32_t material, std::vector<rt_triangle>& tris, std::string& err);
 int hip_error(rt_ctx* ctx, hipError_t e, const char* what);
-enum { kWsRender = 0, kWsStack = 1, kWsStats = 2, kWsSpill = 3, kWsBuild = 4, kWsOrder = 5 };
+enum { kWsRender = 0, kWsStack = 1, kWsStats = 2, kWsBuild = 3, kWsOrder = 4 };
 // Persistent launches take their ray cursors from a ring of blocks; a block
 // holds kSegments counters kCursorStride words apart (one 128-byte line
 // each), one per segment of the ray range.
@@ -303,6 +308,42 @@ int ensure_workspace(rt_ctx* ctx, int slot, size_t bytes);
         if (_e != hipSuccess) return ::rtamd::hip_error((ctx), _e, #call); \
     } while (0)
 
+// How a launch of n rays uses a grid of at most `grid` blocks: the blocks
+// that get rays, and the consecutive rays each of their waves takes at its
+// start -- or 0 for waves that fetch rays from the cursors as they go.
+//
+// A launch lasts as long as its longest ray's chain of record reads, and the
+// lanes a wave has left over take that ray's subtrees from the first step
+// on, so few rays want many waves; but a wave pays for its steps whatever
+// its lanes do, so many rays want full ones, and a CU with one block more
+// than the others holds up the launch.  Waves per SIMD (k) were swept, us
+// per query (262,144-triangle clusters unless said):
+//   rays      16,411  65,536  131,072  262,144  400,000  1,048,576
+//   k = 2       59      92
+//   k = 3       56      87      111      158      196       366
+//   k = 4       58      89      115      147                350
+//   k = 5               95      123      154      206       335
+//   icosphere, 500k rays: camera 153 (4), 165 (5), shell 167 (4), 173 (5)
+//   1,024 triangles: 4,096 rays 20.7 (2), 21.8 (4); 65,536 44.0 (2), 48.3 (5)
+// and at least 4, 8 or 16 rays a wave cost 22.6, 25.0 and 29.8 us against
+// 17.3 on 256 rays: down to one a wave.
+struct LaunchPlan { uint32_t blocks, per_wave; };
+RT_HOST_DEVICE inline LaunchPlan plan_launch(uint32_t n, uint32_t grid, uint32_t waves_per_block, uint32_t simds) {
+    const uint32_t load = n / simds + (n % simds != 0u);           // rays a SIMD
+    uint32_t k = load <= 8u ? 2u : load <= 192u ? 3u : (load + 63u) / 64u;
+    if (load > 320u) k = (load + 64u) / 128u;
+    const uint64_t want = (uint64_t)k * simds / waves_per_block;
+    LaunchPlan p{want < grid ? (uint32_t)want : grid, 0u};
+    // down to one ray a wave, in a number of blocks that the XCDs share evenly
+    const uint32_t most = (n / waves_per_block + (n % waves_per_block != 0u) + kXcds - 1u) / kXcds * kXcds;
+    if (most < p.blocks) p.blocks = most;
+    if (p.blocks == 0u) return p;
+    const uint32_t waves = p.blocks * waves_per_block;
+    const uint32_t per = n / waves + (n % waves != 0u);
+    if (per <= 64u) p.per_wave = per;
+    return p;
+}
+
 // Launchers (rt_trace.hip).
 struct TraceArgs {
     const rt_scene* scene;
@@ -319,8 +360,14 @@ struct TraceArgs {
     bool cursor_zeroed = false;        // an earlier kernel on the stream zeroed cursor's segment words
     unsigned long long* sums = nullptr;   // counting variant: record totals (2 words), or null
     bool no_alloc = false;             // a variant that must not allocate: refuse what would
+    uint32_t expect = 0;               // rays a queue of capacity n is likely to hold (0: n)
 };
 int launch_trace_packed(rt_ctx* ctx, const TraceArgs& a, hipStream_t s);
+// The context's area for stack entries past those in LDS, `entries` deep for
+// every lane of a launch; made on first use, null while `s` is capturing and
+// there is none yet.
+int stack_spill(rt_ctx* ctx, uint32_t entries, hipStream_t s, int32_t** out);
+constexpr int kNoSpill = -1;               // a launch's status: it needs an area it cannot have
 // The next block of the context's ray-cursor ring (kCursorBlock words; the
 // traversal reads word k * kCursorStride of segment k).
 uint32_t* next_cursor(rt_ctx* ctx);
@@ -341,6 +388,8 @@ int noalloc_setup(int device);
 // Idle lanes that make a drained wave share its busy lanes' work
 // (rt_tuning.steal, default 32).
 uint32_t drain_steal(const rt_ctx* ctx);
+// SIMDs of the context's device (plan_launch).
+inline uint32_t device_simds(const rt_ctx* ctx) { return (uint32_t)ctx->num_cus * 4u; }
 int resolved_layout(const rt_ctx* ctx);   // RT_LAYOUT_* actually used
 int launch_trace_reference(rt_ctx* ctx, const TraceArgs& a, uint32_t max_stack, hipStream_t s);
 // Spheres after a traversal (rt_sphere.hip): no-op unless a.spheres is set

@@ -343,6 +343,8 @@ int render_impl(rt_ctx* ctx, const rt_scene* sc, const rt_ubo& ubo, const rt_ren
         TraceArgs ta{sc, rays[b & 1], P, n_dev, hits, prm.spheres, nullptr, nullptr, true};
         if (use_packed) {
             ta.sums = sums;
+            // camera rays fill the queue; about half of them go on
+            ta.expect = b == 0 ? P : (P + 1) / 2;
             ta.cursor = cursor;
             ta.cursor_zeroed = true;
         }

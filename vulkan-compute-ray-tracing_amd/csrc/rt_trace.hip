@@ -28,17 +28,17 @@ namespace rtamd {
 namespace {
 
 // Closest-hit queries (rt_closest_hit, rt_closest_hit_stats).
-template <int BLOCK, int STACK, int LAYOUT, bool STATS, int RING>
+template <int BLOCK, int STACK, int LAYOUT, bool STATS, bool DEEP>
 __global__ __launch_bounds__(BLOCK) void k_trace_packed(TraceScene sc, TraceIo io, int32_t* spill) {
-    __shared__ int32_t stk[(RING ? RING : STACK) * BLOCK];
-    trace_persistent<BLOCK, STACK, LAYOUT, STATS, false, RING>(sc, io, BatchIo{}, stk, spill);
+    __shared__ int32_t stk[STACK * BLOCK];
+    trace_persistent<BLOCK, STACK, LAYOUT, STATS, false, DEEP>(sc, io, BatchIo{}, stk, spill);
 }
 
 // The render's per-bounce traces over the live-ray queue (count on device).
-template <int BLOCK, int STACK, int LAYOUT, int RING>
+template <int BLOCK, int STACK, int LAYOUT, bool DEEP>
 __global__ __launch_bounds__(BLOCK) void k_trace_render(TraceScene sc, TraceIo io, int32_t* spill) {
-    __shared__ int32_t stk[(RING ? RING : STACK) * BLOCK];
-    trace_persistent<BLOCK, STACK, LAYOUT, false, false, RING>(sc, io, BatchIo{}, stk, spill);
+    __shared__ int32_t stk[STACK * BLOCK];
+    trace_persistent<BLOCK, STACK, LAYOUT, false, false, DEEP>(sc, io, BatchIo{}, stk, spill);
 }
 
 // intersectAABB (ray-trace-compute.comp:250-258) with GLSL min/max.
@@ -173,6 +173,23 @@ size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 }  // namespace
 
+// Spill areas are cut in three depths, so a context holds at most three and
+// none is ever replaced (a captured launch keeps its area's address): 16, 32
+// or 96 entries for every lane a launch can have.
+int stack_spill(rt_ctx* ctx, uint32_t entries, hipStream_t s, int32_t** out) {
+    const int k = entries <= 16 ? 0 : entries <= 32 ? 1 : 2;
+    constexpr uint32_t kDepth[3] = {16, 32, kMaxWideStack};
+    *out = nullptr;
+    if (!ctx->d_spill[k]) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (s && hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone) return RT_OK;
+        RT_HIP(ctx, hipMalloc((void**)&ctx->d_spill[k],
+                              sizeof(int32_t) * kDepth[k] * (size_t)ctx->num_cus * kMaxLanesPerCu));
+    }
+    *out = ctx->d_spill[k];
+    return RT_OK;
+}
+
 // Ray cursors for persistent launches: a ring of counters so launches on
 // different streams never share one.  A launch zeroes its block with a fill
 // kernel on its own stream right before use, unless the caller had an
@@ -184,39 +201,34 @@ uint32_t* next_cursor(rt_ctx* ctx) {
 
 namespace {
 
-template <int STACK, int LAYOUT, int RING>
+template <int STACK, int LAYOUT, bool DEEP>
 int launch_packed_t(rt_ctx* ctx, const TraceArgs& a, hipStream_t s, bool stats) {
     const rt_scene* sc = a.scene;
     // the counting variant also serves a render whose record totals are asked for
-    auto kern = stats      ? k_trace_packed<kBlock, STACK, LAYOUT, true, RING>
-                : a.render ? k_trace_render<kBlock, STACK, LAYOUT, RING>
-                           : k_trace_packed<kBlock, STACK, LAYOUT, false, RING>;
+    auto kern = stats      ? k_trace_packed<kBlock, STACK, LAYOUT, true, DEEP>
+                : a.render ? k_trace_render<kBlock, STACK, LAYOUT, DEEP>
+                           : k_trace_packed<kBlock, STACK, LAYOUT, false, DEEP>;
     int per_cu = 0;
     RT_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kBlock, 0));
     if (per_cu < 1) per_cu = 1;
     if (ctx->tuning.blocks_per_cu && (int)ctx->tuning.blocks_per_cu < per_cu) per_cu = (int)ctx->tuning.blocks_per_cu;
     uint32_t blocks = (uint32_t)ctx->num_cus * (uint32_t)per_cu;
+    const uint32_t simds = device_simds(ctx);
+    bool cursors = true;               // read by this launch (a render's queue length is on the device)
     if (!a.n_dev) {
-        // no more waves than rays: down to one ray a wave, whose other lanes
-        // take its subtrees (trace_persistent, drain).  At least 4, 8, 16 or
-        // 32 rays a wave measured 22.6, 25.0, 29.8 and 33.1 us against 17.3
-        // on 256 rays and 1,024 triangles, 38, 48, 57 and 70 against 31 on
-        // 1,000 rays and 262,144 triangles, and the same from 64k rays up
-        const uint32_t need = (a.n - 1) / (kBlock / 64) + 1;
         if (a.n == 0) return RT_OK;
-        if (need < blocks) blocks = need;
+        const LaunchPlan plan = plan_launch(a.n, blocks, kBlock / 64, simds);
+        blocks = plan.blocks;
+        cursors = plan.per_wave == 0;
     }
     int32_t* spill = nullptr;
-    if (RING) {
-        if (a.no_alloc)
-            return set_error(ctx, RT_ERR_UNSUPPORTED, "an LDS stack ring spills to a workspace: set stack_lds to 0");
-        int rc = ensure_workspace(ctx, kWsSpill, (size_t)(STACK - RING) * blocks * kBlock * sizeof(int32_t));
+    if (DEEP) {
+        const int rc = stack_spill(ctx, sc->stack4 - STACK, s, &spill);
         if (rc) return rc;
-        spill = (int32_t*)ctx->ws[kWsSpill];
+        if (!spill) return kNoSpill;
     }
     uint32_t* cursor = a.cursor ? a.cursor : next_cursor(ctx);
-    // a launch with a lane for every ray reads no cursor
-    if (!(a.cursor && a.cursor_zeroed) && (a.n_dev || a.n > (uint64_t)blocks * kBlock)) {
+    if (cursors && !(a.cursor && a.cursor_zeroed)) {
         const int rc = launch_fill_u32(ctx, cursor, 0u, kCursorBlock, s);
         if (rc) return rc;
     }
@@ -240,7 +252,7 @@ int launch_packed_t(rt_ctx* ctx, const TraceArgs& a, hipStream_t s, bool stats) 
     TraceScene ts{sc->d_pnodes, sc->d_qnodes, sc->d_w4nodes, sc->d_ptris, sc->d_ptri_id, sc->frame,
                   LAYOUT == kLayoutW4 || LAYOUT == kLayoutW4Joined ? sc->root4 : sc->root_ref, sc->tri_off};
     TraceIo io{a.rays, a.n_dev, a.hits, a.node_visits, a.tri_tests, cursor, a.n, refill, a.order, segs,
-               drain_steal(ctx), a.sums};
+               drain_steal(ctx), simds, a.sums};
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), 0, s, ts, io, spill);
     RT_HIP(ctx, hipGetLastError());
     return RT_OK;
@@ -248,18 +260,15 @@ int launch_packed_t(rt_ctx* ctx, const TraceArgs& a, hipStream_t s, bool stats) 
 
 template <int STACK>
 int launch_packed_layout(rt_ctx* ctx, const TraceArgs& a, hipStream_t s, bool stats) {
-    if (ctx->tuning.node_layout == RT_LAYOUT_F32) return launch_packed_t<STACK, kLayoutF32, 0>(ctx, a, s, stats);
-    return launch_packed_t<STACK, kLayoutQ16, 0>(ctx, a, s, stats);
+    if (ctx->tuning.node_layout == RT_LAYOUT_F32) return launch_packed_t<STACK, kLayoutF32, false>(ctx, a, s, stats);
+    return launch_packed_t<STACK, kLayoutQ16, false>(ctx, a, s, stats);
 }
 
-template <int STACK>
+// 4-wide records: STACK entries in LDS, the rest (DEEP) in the context's spill area.
+template <int STACK, bool DEEP>
 int launch_w4(rt_ctx* ctx, const TraceArgs& a, hipStream_t s, bool stats) {
-    const uint32_t ring = ctx->tuning.stack_lds;
-    if (ring == 8 && STACK > 8) return launch_packed_t<STACK, kLayoutW4, 8>(ctx, a, s, stats);
-    if (ring == 32 && STACK > 32) return launch_packed_t<STACK, kLayoutW4, 32>(ctx, a, s, stats);
-    if (ring == 16 && STACK > 16) return launch_packed_t<STACK, kLayoutW4, 16>(ctx, a, s, stats);
-    if (a.scene->tri_off != kSeparateArrays) return launch_packed_t<STACK, kLayoutW4Joined, 0>(ctx, a, s, stats);
-    return launch_packed_t<STACK, kLayoutW4, 0>(ctx, a, s, stats);
+    if (a.scene->tri_off != kSeparateArrays) return launch_packed_t<STACK, kLayoutW4Joined, DEEP>(ctx, a, s, stats);
+    return launch_packed_t<STACK, kLayoutW4, DEEP>(ctx, a, s, stats);
 }
 
 }  // namespace
@@ -342,6 +351,11 @@ int ray_order_in(rt_ctx* ctx, const TraceArgs& a, hipStream_t s, char* ws, size_
     return RT_OK;
 }
 
+namespace {
+// Blocks of kBlock lanes whose whole stacks of `need` entries fit a CU's LDS together.
+uint32_t whole_stack_blocks(uint32_t need) { return need <= kStackLds ? 5u : need <= 36 ? 4u : need <= 48 ? 3u : need <= 64 ? 2u : 1u; }
+}  // namespace
+
 // The sorted order of a query's rays in ctx's order workspace, or null when
 // the batch keeps index order.
 int ray_order(rt_ctx* ctx, const TraceArgs& a, hipStream_t s, const uint32_t** order) {
@@ -359,12 +373,36 @@ int launch_trace_packed(rt_ctx* ctx, const TraceArgs& a, hipStream_t s) {
     const bool stats = (a.node_visits && a.tri_tests) || a.sums;
     if (resolved_layout(ctx) == RT_LAYOUT_W4) {
         const uint32_t need = sc->stack4;
-        if (need <= 24) return launch_w4<24>(ctx, a, s, stats);
-        if (need <= 36) return launch_w4<36>(ctx, a, s, stats);
-        if (need <= 48) return launch_w4<48>(ctx, a, s, stats);
-        if (need <= 64) return launch_w4<64>(ctx, a, s, stats);
-        if (need <= 96) return launch_w4<96>(ctx, a, s, stats);
-        return set_error(ctx, RT_ERR_UNSUPPORTED, "4-wide tree deeper than 31 levels");
+        if (need > kMaxWideStack) return set_error(ctx, RT_ERR_UNSUPPORTED, "4-wide tree deeper than 31 levels");
+        // Where the blocks this launch wants on a CU fit with whole stacks in
+        // LDS, they stay there; else the first kStackLds entries do, and five
+        // blocks fit (five is also what 92 VGPRs allow).  The 4M-triangle
+        // tree needs 46 entries: three whole-stack blocks of 48 entries take
+        // 3.30 ms for 4M rays, four of 40 (most rays never go deeper) 3.06,
+        // five of 24 2.70; a sixth block would cost 13 spilled registers and
+        // takes 3.51.  But at equal blocks the depth test costs 1-4%
+        // (131,072 rays on 262,144 triangles: 117 us against 111).
+        const uint32_t cus = (uint32_t)ctx->num_cus;
+        const uint32_t expect = a.expect ? a.expect : a.n;
+        const uint32_t want = (plan_launch(expect, cus * 5u, kBlock / 64, device_simds(ctx)).blocks + cus - 1u) / cus;
+        const uint32_t lds = ctx->tuning.stack_lds;
+        int rc = kNoSpill;
+        if (lds && lds < need) {
+            if (a.no_alloc)
+                return set_error(ctx, RT_ERR_UNSUPPORTED, "a partial LDS stack spills to a workspace: set stack_lds to 0");
+            if (lds == 8) rc = launch_w4<8, true>(ctx, a, s, stats);
+            else if (lds == 16) rc = launch_w4<16, true>(ctx, a, s, stats);
+            else rc = launch_w4<32, true>(ctx, a, s, stats);
+        } else if (need > kStackLds && want > whole_stack_blocks(need) && !a.no_alloc) {
+            rc = launch_w4<kStackLds, true>(ctx, a, s, stats);
+        }
+        // (no spill area during a capture that comes before the area exists)
+        if (rc != kNoSpill) return rc;
+        if (need <= kStackLds) return launch_w4<kStackLds, false>(ctx, a, s, stats);
+        if (need <= 36) return launch_w4<36, false>(ctx, a, s, stats);
+        if (need <= 48) return launch_w4<48, false>(ctx, a, s, stats);
+        if (need <= 64) return launch_w4<64, false>(ctx, a, s, stats);
+        return launch_w4<kMaxWideStack, false>(ctx, a, s, stats);
     }
     // binary records are built on first use (an upload under the 4-wide
     // layout leaves them out); the scene's arrays are immutable otherwise

@@ -223,6 +223,7 @@ struct TraceIo {
     const uint32_t* order;    // trace order (ray indices), or null: index order
     uint32_t segs;            // segments of the ray range (1 or kSegments), see below
     uint32_t steal;           // idle lanes that make a drained wave share work (65: never)
+    uint32_t simds;           // SIMDs of the device (plan_launch)
     unsigned long long* sums; // counting variant: totals of node and triangle records, or null
 };
 
@@ -274,9 +275,10 @@ __device__ __forceinline__ float shfl_f(float x, uint32_t src) {
 // outside the frame, whose node tests run on t - t_shift (frame_far).
 //
 // BATCHED: rays come from many items (BatchIo); each lane carries its own
-// scene pointers.  RING > 0: only the top RING stack entries of a lane live
-// in LDS (a ring); deeper entries move to `spill` in HBM, one word per
-// push/pop beyond RING.  RING = 0 keeps the whole stack (STACK entries) in LDS.
+// scene pointers.  A lane's stack has its first STACK entries in LDS; with
+// DEEP, entries past those go to `spill` in HBM ([entry - STACK][lane of the
+// grid]), which few rays ever reach.  Without DEEP the host has checked that
+// the scenes need no more than STACK.
 //
 // Work sharing in the drain (4-wide layouts, whole stack in LDS, no
 // counters; in batched launches the helper also takes the donor's scene):
@@ -298,15 +300,17 @@ __device__ __forceinline__ float shfl_f(float x, uint32_t src) {
 // 0, with its closest t as an inclusive bound: only boxes up to that t are
 // visited, in the order of a full traversal (a child's place among its
 // siblings depends on entry distances alone), and the first hit met is kept.
-template <int BLOCK, int STACK, int LAYOUT, bool STATS, bool BATCHED, int RING>
+template <int BLOCK, int STACK, int LAYOUT, bool STATS, bool BATCHED, bool DEEP>
 __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const TraceIo& io, const BatchIo& bio,
                                                  int32_t* __restrict__ stk, int32_t* __restrict__ spill) {
     static_assert(!BATCHED || LAYOUT == kLayoutW4 || LAYOUT == kLayoutQ16,
                   "batched launches read 4-wide or binary 16-bit records");
     constexpr bool kW4 = LAYOUT == kLayoutW4 || LAYOUT == kLayoutW4Joined;
-    constexpr bool STEAL = kW4 && RING == 0 && !STATS;
-    static_assert(RING == 0 || (RING & (RING - 1)) == 0, "ring size is a power of two");
+    constexpr bool STEAL = kW4 && !STATS;
     const uint32_t n = io.n_dev ? *io.n_dev : io.n_host;
+    const LaunchPlan plan = plan_launch(n, gridDim.x, BLOCK / 64, io.simds);
+    if (blockIdx.x >= plan.blocks) return;
+    const bool fits = plan.per_wave != 0u;      // rays handed out once, without cursors
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = lane_id();
     const uint64_t lanes_below = (1ull << lane) - 1ull;
@@ -329,18 +333,6 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                        ? (blockIdx.x % kXcds) * (kSegments / kXcds) + (blockIdx.x / kXcds) % (kSegments / kXcds)
                        : (uint32_t)(blockIdx.x % io.segs);
     uint32_t tried = 0;
-    // A launch with a lane for every ray hands them out once, without
-    // cursors, and evenly over the grid's waves: rays_per_wave consecutive
-    // ones each.  Blocks of one XCD take one run of the rays.  Such a launch
-    // lasts as long as its longest ray's chain of record reads, so it wants
-    // few rays in a wave: the lanes left over take subtrees from the start
-    // (the drain below).  Full waves from a cursor took 43.7 us where this
-    // takes 17.3 on 256 rays and 1,024 triangles, 104.9 against 55.6 on
-    // 16,411 rays and 262,144 triangles, and 793.7 against 454.4 on a
-    // 512 x 512 render of four bounces.
-    const uint32_t waves = gridDim.x * (BLOCK / 64);
-    const bool fits = n <= waves * 64u;
-    const uint32_t rays_per_wave = (n + waves - 1u) / waves;
     // the segment's ray range [seg_lo, seg_hi); io.segs is 1 or kSegments,
     // both powers of two, so the bounds are a product and a shift
     const uint32_t seg_shift = io.segs == kSegments ? kSegmentShift : 0u;
@@ -390,22 +382,23 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
     const int32_t* l_triid = sc.tri_id;
     rt_hit* l_hits = io.hits;
 
-    auto push = [&](int32_t v) {
-        if (RING == 0) {
-            stk[sp * BLOCK + tid] = v;
-        } else {
-            const int slot = sp & (RING - 1);
-            if (sp >= RING) spill[(size_t)(sp - RING) * gstride + gtid] = stk[slot * BLOCK + tid];
-            stk[slot * BLOCK + tid] = v;
-        }
+    // `deep` is uniform: whether any lane may touch an entry past STACK in
+    // this step.  Testing that once a step, rather than each entry, keeps the
+    // usual path as short as without DEEP.
+    auto push = [&](int32_t v, bool deep) {
+        if (!deep || sp < STACK) stk[sp * BLOCK + tid] = v;
+        else spill[(size_t)(sp - STACK) * gstride + gtid] = v;
         sp++;
     };
-    auto pop = [&]() -> int32_t {
+    auto pop = [&](bool deep) -> int32_t {
         sp--;
-        if (RING == 0) return stk[sp * BLOCK + tid];
-        const int slot = sp & (RING - 1);
-        int32_t v = stk[slot * BLOCK + tid];
-        if (sp >= RING) stk[slot * BLOCK + tid] = spill[(size_t)(sp - RING) * gstride + gtid];
+        if (!deep) return stk[sp * BLOCK + tid];
+        int32_t v = 0;
+        if (sp < STACK) v = stk[sp * BLOCK + tid];
+        else v = spill[(size_t)(sp - STACK) * gstride + gtid];
+        // waited for here: in flight past the join it would make every next
+        // step wait for all outstanding memory operations, hit stores too
+        asm volatile("" : "+v"(v));
         return v;
     };
 
@@ -413,6 +406,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
     auto step = [&](auto sh) {
         constexpr bool SH = decltype(sh)::value;
         if (!busy) return;
+        const bool deep = DEEP && __ballot(sp > STACK - 3) != 0;
         bool next = false;          // cur holds the next record to read
         if (sp >= 0 && kW4) {
             // One memory round trip per step whatever the lanes' mix of
@@ -483,9 +477,15 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                     cswap(k1, v1, k3, v3);
                     cswap(k1, v1, k2, v2);
                     // farthest pushed first so the nearest deferred child pops first
-                    if (nh > 3) push(v3);
-                    if (nh > 2) push(v2);
-                    if (nh > 1) push(v1);
+                    if (deep) {
+                        if (nh > 3) push(v3, true);
+                        if (nh > 2) push(v2, true);
+                        if (nh > 1) push(v1, true);
+                    } else {
+                        if (nh > 3) push(v3, false);
+                        if (nh > 2) push(v2, false);
+                        if (nh > 1) push(v1, false);
+                    }
                     cur = v0;
                     next = true;
                 }
@@ -536,7 +536,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                 if (STATS) nv++;
                 if (h0 && h1) {
                     bool swap = tn1 < tn0;
-                    push(swap ? c0 : c1);
+                    push(swap ? c0 : c1, false);
                     cur = swap ? c1 : c0;
                     next = true;
                 } else if (h0 || h1) {
@@ -557,7 +557,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
         }
         if (!next) {
             if (sp > (SH ? bot : 0)) {
-                cur = pop();
+                cur = pop(deep);
             } else if (SH && owner >= 0) {
                 handoff = true;             // a helper's part is done
                 busy = false;
@@ -594,11 +594,13 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
             uint32_t lo = seg_lo, hi = seg_hi;
             uint32_t base = 0;
             if (fits) {
-                const uint32_t b = gridDim.x % kXcds == 0
-                                       ? (blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds : blockIdx.x;
-                const uint64_t first = (uint64_t)(b * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(tid / 64u)) * rays_per_wave;
+                // one run of rays to the blocks of each XCD
+                const uint32_t b = plan.blocks % kXcds == 0
+                                       ? (blockIdx.x % kXcds) * (plan.blocks / kXcds) + blockIdx.x / kXcds : blockIdx.x;
+                const uint64_t first =
+                    (uint64_t)(b * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(tid / 64u)) * plan.per_wave;
                 lo = (uint32_t)(first < n ? first : n);
-                hi = n - lo > rays_per_wave ? lo + rays_per_wave : n;
+                hi = n - lo > plan.per_wave ? lo + plan.per_wave : n;
                 drained = true;
             } else if (lane == leader) {
                 base = atomicAdd(io.cursor + (size_t)seg * kCursorStride, n_idle);
@@ -691,7 +693,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                 const float owner_rel = shfl_f(best_rel, owner < 0 ? lane : (uint32_t)owner);
                 if (busy && owner >= 0) best_rel = fminf(best_rel, owner_rel);
                 const uint64_t idle_m = __ballot(!busy && !waiting);
-                const uint64_t donor_m = __ballot(busy && !exact && sp - bot >= 1);
+                const uint64_t donor_m = __ballot(busy && !exact && sp - bot >= 1 && (!DEEP || bot < STACK));
                 if ((uint32_t)__popcll(idle_m) >= io.steal && donor_m != 0) {
                     const uint32_t k = min((uint32_t)__popcll(idle_m), (uint32_t)__popcll(donor_m));
                     const uint32_t rank_idle = (uint32_t)__popcll(idle_m & lanes_below);
@@ -732,7 +734,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                             l_tris = reinterpret_cast<const PTri*>(v_tris);
                             l_triid = reinterpret_cast<const int32_t*>(v_triid);
                         }
-                        // the donor's bottom entry: v_bot < donor's sp <= STACK
+                        // the donor's bottom entry, in LDS: v_bot < STACK
                         cur = stk[v_bot * BLOCK + (int)(tid - lane + src)];
                         r.o = f3{ox, oy, oz};
                         r.d = f3{dx, dy, dz};
