@@ -75,8 +75,12 @@ struct alignas(16) PNode4 { uint32_t w[12]; int32_t ref[4]; };
 static_assert(sizeof(PNode4) == 64, "4-wide node record");
 constexpr int32_t kNoChild = INT32_MIN + 1;
 
-// Fixed-point frame of the quantized nodes, with 1/scale for the rays.
-struct QFrame { float ox, oy, oz, sx, sy, sz, rx, ry, rz; };
+// Fixed-point frame of the quantized nodes, with 1/scale for the rays in
+// binary32 and binary64 (a ray's setup takes products, not divisions).
+struct QFrame {
+    float ox, oy, oz, sx, sy, sz, rx, ry, rz;
+    double dx, dy, dz;
+};
 
 // kLayoutW4Joined is kLayoutW4 with its records and packed triangles in one
 // allocation (rt_scene::tri_off), addressed by 32-bit offsets.
@@ -295,6 +299,8 @@ constexpr uint32_t kSegments = 8;               // one segment per XCD (32, four
 constexpr uint32_t kSegmentShift = 3;           // log2(kSegments)
 static_assert(kSegments == 1u << kSegmentShift, "segments are a power of two");
 constexpr uint32_t kCursorStride = 32;
+constexpr uint32_t kChunkRays = 64;             // rays a wave takes from a cursor at once,
+constexpr uint32_t kChunkedRays = 192;          // where there are this many for each wave
 constexpr uint32_t kCursorBlock = kSegments * kCursorStride;
 constexpr uint32_t kCursorBlocks = 256;
 // A render's per-bounce counters (rt_ctx::d_counters): [b] = live rays entering bounce b.

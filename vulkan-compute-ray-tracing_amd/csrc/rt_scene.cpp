@@ -280,7 +280,8 @@ void quantize_nodes(PackedTree& out) {
         org[k] = (float)(lo[k] - 2.0 * (double)scl[k]);
         if ((double)org[k] > lo[k] - 2.0 * (double)scl[k]) org[k] = std::nextafter(org[k], -INFINITY);
     }
-    out.frame = QFrame{org[0], org[1], org[2], scl[0], scl[1], scl[2], 1.0f / scl[0], 1.0f / scl[1], 1.0f / scl[2]};
+    out.frame = QFrame{org[0], org[1], org[2], scl[0], scl[1], scl[2], 1.0f / scl[0], 1.0f / scl[1], 1.0f / scl[2],
+                       1.0 / (double)scl[0], 1.0 / (double)scl[1], 1.0 / (double)scl[2]};
     // q covers [org + q*scl] exactly (double arithmetic of the float frame)
     auto qlo = [&](float v, int k) -> uint32_t {
         double q = std::floor(((double)v - (double)org[k]) / (double)scl[k]) - 1.0;
