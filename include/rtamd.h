@@ -134,7 +134,9 @@ const char* rt_last_error(const rt_ctx* ctx);
 const char* rt_status_string(int status);
 
 /* Copies the arrays into HBM, validates indices and the tree, and repacks
- * nodes/triangles for traversal.  Replaces the six BufferUtils::createBundle
+ * nodes/triangles for traversal.  Scratch for that, about 350 bytes a
+ * triangle, is given back before the call returns, but for up to 256 MiB
+ * that the context keeps.  Replaces the six BufferUtils::createBundle
  * uploads (main.cpp:84-106, Buffer.h:83-102) and ComputeMaterial::init
  * (ComputeMaterial.cpp:15-26).  Counts are whole-array counts (the shader's
  * .length()), not the one-element descriptor range of Buffer.h:85.  An empty
@@ -446,8 +448,9 @@ int rt_host_alloc(size_t bytes, void** out);
 int rt_host_free(void* p);
 int rt_server_create(rt_ctx* ctx, const rt_server_config* config, rt_server** out);
 int rt_server_destroy(rt_server* server);
-/* Makes a scene resident.  Admission comes before any device allocation:
- * the scene is validated and packed on the host, which fixes its device
+/* Makes a scene resident.  Admission comes before the scene's own device
+ * memory: it is validated and packed first (in the upload's scratch, or on
+ * the host), which fixes its device
  * bytes; least recently used idle scenes are then evicted (and freed) while
  * the budget, or the device's free memory, cannot hold it, and only then is
  * it uploaded -- resident bytes never exceed the budget, not even during a

@@ -325,7 +325,7 @@ size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 }  // namespace
 }  // namespace rtamd
 
-#include "rt_wide.hpp"
+#include "rt_pack.hpp"
 
 using namespace rtamd;
 

@@ -151,6 +151,7 @@ void widen_nodes(PackedTree& out);
 // that fixes its size and the emission into the scene's arrays.
 struct WideTree;
 struct WideTreeDelete { void operator()(WideTree* t) const; };
+constexpr uint32_t kMaxPackedHeight = 64;  // binary levels of a packed tree
 constexpr uint32_t kMaxWideStack = 96;     // deepest stack a traversal may need
 constexpr uint32_t kStackLds = 24;         // entries of a lane's stack in LDS, 4-wide layout
 constexpr uint32_t kMaxLanesPerCu = 2048;  // of any launch: 8 waves on each of 4 SIMDs
@@ -164,6 +165,13 @@ int wide_build(rt_ctx* ctx, const PackedTree& packed, hipStream_t s, std::unique
 // Writes the caller's records (nodes[0..), leaf refs moved), the device
 // tree's after them (its root first), and the triangles and their ids in its order.
 int wide_emit(rt_ctx* ctx, const WideTree& t, uint32_t records, PNode4* nodes, PTri* tris, int32_t* ids, hipStream_t s);
+// The caller's arrays on the device (a scene packed there), else null.
+const rt_triangle* wide_triangles(const WideTree& t);
+const rt_bvh_node* wide_nodes(const WideTree& t);
+// Uploads up to this much scratch keep it in the context (kWsUpload).
+constexpr size_t kUploadKept = 256u << 20;
+// The 16-bit frame of boxes whose bounds are [lo, hi].
+QFrame quant_frame(const double lo[3], const double hi[3]);
 
 }  // namespace rtamd
 
@@ -182,9 +190,10 @@ constexpr uint32_t kSphereLinear = 16;     // up to this many: a plain loop
 constexpr uint32_t kSphereStack = 32;      // LDS stack entries per lane
 constexpr uint32_t kMaxTreeSpheres = 1u << 24;   // median split: depth <= 24
 
-// Host half of an upload: the scene validated and packed, its device bytes
-// known before anything is allocated on the device (so a caller with an
-// HBM budget can make room first).  scene_commit allocates and copies.
+// First half of an upload: the scene validated and packed, in scratch on the
+// device or on the host, its device bytes known before any of them is
+// allocated (so a caller with an HBM budget can make room first).
+// scene_commit allocates and copies.
 struct PreparedScene {
     rt_scene_desc desc{};               // the caller's arrays (the tree the shader order walks)
     std::vector<rt_bvh_node> built;     // the device-built tree (RT_TREE_DEVICE), or empty
@@ -197,14 +206,20 @@ struct PreparedScene {
     bool with_pnodes = false, with_qnodes = false;   // binary records uploaded now
     std::unique_ptr<WideTree, WideTreeDelete> wide;  // the tree the 4-wide traversal walks, or null: the caller's
     uint32_t wide_records = 0, wide_need = 0;
+    // packed by device_pack: `packed` holds only the frame, roots and depths,
+    // and the caller's arrays are on the device already
+    bool device_packed = false;
+    uint32_t given_records = 0, leaf_slots = 0;      // the caller's 4-wide records and the triangle slots
     uint64_t bytes = 0;                 // device bytes scene_commit allocates
 };
-int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& out);
+// `plain`: on the host, without a tree of its own (needs no device memory).
+int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& out, bool plain = false);
 int scene_commit(rt_ctx* ctx, PreparedScene& prep, rt_scene** out);
-// Gives the prepared device tree and its scratch back; P.bytes follows.
-void scene_drop_wide(PreparedScene& P);
-// Device bytes of the 4-wide records (the device tree's `wide` among them) and packed triangles as uploaded.
-uint64_t packed_record_bytes(const PackedTree& p, uint32_t wide);
+// Validates and packs `d` on the device (rt_pack.hpp); *done stays false
+// where the host has to.
+int device_pack(rt_ctx* ctx, const rt_scene_desc& d, PreparedScene& P, bool* done);
+// Device bytes of 4-wide records and packed triangles as uploaded.
+uint64_t packed_record_bytes(uint64_t records, uint64_t slots);
 // The binary node records of `layout` (RT_LAYOUT_F32 / RT_LAYOUT_Q16) for a
 // scene uploaded without them: rebuilt from the scene's device arrays.
 int scene_binary_records(rt_ctx* ctx, rt_scene* s, uint32_t layout);
@@ -218,6 +233,9 @@ struct rt_scene {
     rt_bvh_node* d_nodes = nullptr;
     rt_light* d_lights = nullptr;
     rt_sphere* d_spheres = nullptr;
+    // the arrays above, d_snodes and d_ptri_id are parts of this one allocation
+    // (a scene packed on the device), or allocations of their own when it is null
+    char* d_base = nullptr;
     rtamd::PNode* d_pnodes = nullptr;
     rtamd::PNodeQ* d_qnodes = nullptr;
     rtamd::PNode4* d_w4nodes = nullptr;
@@ -254,8 +272,8 @@ struct rt_ctx {
     int num_cus = 0;
     // grow-only device workspaces: [0] render path state, [1] reference
     // traversal stacks, [2] statistics scratch, [3] BVH builder scratch,
-    // [4] ray-order keys and permutation
-    static constexpr int kWorkspaces = 5;
+    // [4] ray-order keys and permutation, [5] upload scratch
+    static constexpr int kWorkspaces = 6;
     void* ws[kWorkspaces] = {};
     size_t ws_bytes[kWorkspaces] = {};
     int32_t* d_spill[3] = {};         // stack entries past LDS (stack_spill), each made on first use
@@ -290,7 +308,7 @@ int set_error(rt_ctx* ctx, int code, const std::string& msg);
 // Triangles of one OBJ file (rt_obj.cpp); err receives the reason on failure.
 int obj_triangles(const char* path, uint32_t material, std::vector<rt_triangle>& tris, std::string& err);
 int hip_error(rt_ctx* ctx, hipError_t e, const char* what);
-enum { kWsRender = 0, kWsStack = 1, kWsStats = 2, kWsBuild = 3, kWsOrder = 4 };
+enum { kWsRender = 0, kWsStack = 1, kWsStats = 2, kWsBuild = 3, kWsOrder = 4, kWsUpload = 5 };
 // Persistent launches take their ray cursors from a ring of blocks; a block
 // holds kSegments counters kCursorStride words apart (one 128-byte line
 // each), one per segment of the ray range.

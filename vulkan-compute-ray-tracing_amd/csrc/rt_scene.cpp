@@ -256,17 +256,7 @@ void widen_nodes(PackedTree& out) {
     }
 }
 
-void quantize_nodes(PackedTree& out) {
-    out.qnodes.assign(out.nodes.size(), PNodeQ{});
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (const PNode& p : out.nodes) {
-        const float c[12] = {p.a.x, p.a.y, p.a.z, p.a.w, p.b.x, p.b.y, p.b.z, p.b.w, p.c.x, p.c.y, p.c.z, p.c.w};
-        for (int k = 0; k < 3; ++k) {
-            lo[k] = std::min(lo[k], (double)std::min(c[k], c[6 + k]));
-            hi[k] = std::max(hi[k], (double)std::max(c[3 + k], c[9 + k]));
-        }
-    }
-    if (out.nodes.empty()) for (int k = 0; k < 3; ++k) lo[k] = hi[k] = 0.0;
+QFrame quant_frame(const double lo[3], const double hi[3]) {
     // The frame puts the scene's lowest bound 2 quanta above the origin and
     // its highest at most 65002 quanta above, so every quantized bound
     // (rounded outward by one extra quantum below) lies strictly inside
@@ -280,8 +270,24 @@ void quantize_nodes(PackedTree& out) {
         org[k] = (float)(lo[k] - 2.0 * (double)scl[k]);
         if ((double)org[k] > lo[k] - 2.0 * (double)scl[k]) org[k] = std::nextafter(org[k], -INFINITY);
     }
-    out.frame = QFrame{org[0], org[1], org[2], scl[0], scl[1], scl[2], 1.0f / scl[0], 1.0f / scl[1], 1.0f / scl[2],
-                       1.0 / (double)scl[0], 1.0 / (double)scl[1], 1.0 / (double)scl[2]};
+    return QFrame{org[0], org[1], org[2], scl[0], scl[1], scl[2], 1.0f / scl[0], 1.0f / scl[1], 1.0f / scl[2],
+                  1.0 / (double)scl[0], 1.0 / (double)scl[1], 1.0 / (double)scl[2]};
+}
+
+void quantize_nodes(PackedTree& out) {
+    out.qnodes.assign(out.nodes.size(), PNodeQ{});
+    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+    for (const PNode& p : out.nodes) {
+        const float c[12] = {p.a.x, p.a.y, p.a.z, p.a.w, p.b.x, p.b.y, p.b.z, p.b.w, p.c.x, p.c.y, p.c.z, p.c.w};
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = std::min(lo[k], (double)std::min(c[k], c[6 + k]));
+            hi[k] = std::max(hi[k], (double)std::max(c[3 + k], c[9 + k]));
+        }
+    }
+    if (out.nodes.empty()) for (int k = 0; k < 3; ++k) lo[k] = hi[k] = 0.0;
+    out.frame = quant_frame(lo, hi);
+    const float org[3] = {out.frame.ox, out.frame.oy, out.frame.oz};
+    const float scl[3] = {out.frame.sx, out.frame.sy, out.frame.sz};
     // q covers [org + q*scl] exactly (double arithmetic of the float frame)
     auto qlo = [&](float v, int k) -> uint32_t {
         double q = std::floor(((double)v - (double)org[k]) / (double)scl[k]) - 1.0;
@@ -312,8 +318,6 @@ void quantize_nodes(PackedTree& out) {
 using namespace rtamd;
 
 namespace {
-constexpr uint32_t kMaxPackedHeight = 64;
-
 template <typename T>
 int upload_array(rt_ctx* ctx, T** dst, const T* src, uint32_t n, uint64_t& bytes) {
     *dst = nullptr;
@@ -325,44 +329,50 @@ int upload_array(rt_ctx* ctx, T** dst, const T* src, uint32_t n, uint64_t& bytes
     return RT_OK;
 }
 
-// The 4-wide node records and the packed triangles, in one allocation when
+// Room for 4-wide node records and packed triangles, in one allocation when
 // they fit in 4 GiB (nodes first, triangles from the next 256-byte boundary;
 // the traversal then addresses both by 32-bit offsets from one base), else
 // in two.
-// The triangles' ids (d_ptri_id) go with them.
-int upload_records(rt_ctx* ctx, rt_scene* s, const PreparedScene& P, uint64_t& bytes) {
-    const PackedTree& packed = P.packed;
-    const size_t records = packed.w4nodes.size() + (P.wide ? P.wide_records : 0u);
+int alloc_records(rt_ctx* ctx, rt_scene* s, size_t records, size_t slots, uint64_t& bytes) {
     const size_t nb = (sizeof(PNode4) * records + 255) / 256 * 256;
-    const size_t tb = sizeof(PTri) * packed.tris.size(), ib = sizeof(int32_t) * packed.tri_id.size();
-    if (!records || !tb) {                                   // a single triangle, or none
-        int rc = upload_array(ctx, &s->d_ptris, packed.tris.data(), (uint32_t)packed.tris.size(), bytes);
-        if (!rc) rc = upload_array(ctx, &s->d_ptri_id, packed.tri_id.data(), (uint32_t)packed.tri_id.size(), bytes);
-        return rc;
-    }
+    const size_t tb = sizeof(PTri) * slots;
     if (nb + tb >= (1ull << 32)) {
         RT_HIP(ctx, hipMalloc((void**)&s->d_w4nodes, sizeof(PNode4) * records));
         RT_HIP(ctx, hipMalloc((void**)&s->d_ptris, tb));
         bytes += sizeof(PNode4) * records + tb;
-    } else {
-        char* base = nullptr;
-        RT_HIP(ctx, hipMalloc((void**)&base, nb + tb));
-        s->d_w4nodes = reinterpret_cast<PNode4*>(base);      // owns the allocation
-        s->d_ptris = reinterpret_cast<PTri*>(base + nb);
-        s->tri_off = (uint32_t)nb;
-        bytes += nb + tb;
+        return RT_OK;
     }
+    char* base = nullptr;
+    RT_HIP(ctx, hipMalloc((void**)&base, nb + tb));
+    s->d_w4nodes = reinterpret_cast<PNode4*>(base);          // owns the allocation
+    s->d_ptris = reinterpret_cast<PTri*>(base + nb);
+    s->tri_off = (uint32_t)nb;
+    bytes += nb + tb;
+    return RT_OK;
+}
+
+// The records, triangles and their ids (d_ptri_id) of a scene packed on the host.
+int upload_records(rt_ctx* ctx, rt_scene* s, const PreparedScene& P, uint64_t& bytes) {
+    const PackedTree& packed = P.packed;
+    if (packed.w4nodes.empty() || packed.tris.empty()) {     // a single triangle, or none
+        int rc = upload_array(ctx, &s->d_ptris, packed.tris.data(), (uint32_t)packed.tris.size(), bytes);
+        if (!rc) rc = upload_array(ctx, &s->d_ptri_id, packed.tri_id.data(), (uint32_t)packed.tri_id.size(), bytes);
+        return rc;
+    }
+    int rc = alloc_records(ctx, s, packed.w4nodes.size() + P.wide_records, packed.tris.size(), bytes);
+    if (rc) return rc;
+    const size_t ib = sizeof(int32_t) * packed.tri_id.size();
     RT_HIP(ctx, hipMalloc((void**)&s->d_ptri_id, ib));
     bytes += ib;
     if (P.wide) {
-        const int rc = wide_emit(ctx, *P.wide, P.wide_records, s->d_w4nodes, s->d_ptris, s->d_ptri_id, nullptr);
+        rc = wide_emit(ctx, *P.wide, P.wide_records, s->d_w4nodes, s->d_ptris, s->d_ptri_id, nullptr);
         if (rc) return rc;
         // any stream may trace the scene once the upload returns
         RT_HIP(ctx, hipStreamSynchronize(nullptr));
         return RT_OK;
     }
     RT_HIP(ctx, hipMemcpy(s->d_w4nodes, packed.w4nodes.data(), sizeof(PNode4) * packed.w4nodes.size(), hipMemcpyHostToDevice));
-    RT_HIP(ctx, hipMemcpy(s->d_ptris, packed.tris.data(), tb, hipMemcpyHostToDevice));
+    RT_HIP(ctx, hipMemcpy(s->d_ptris, packed.tris.data(), sizeof(PTri) * packed.tris.size(), hipMemcpyHostToDevice));
     RT_HIP(ctx, hipMemcpy(s->d_ptri_id, packed.tri_id.data(), ib, hipMemcpyHostToDevice));
     return RT_OK;
 }
@@ -461,6 +471,16 @@ bool build_sphere_tree(const rt_sphere* sp, uint32_t n, std::vector<SphereNode>&
 
 void free_scene(rt_scene* s) {
     if (!s) return;
+    if (s->d_base) {
+        (void)hipFree(s->d_base);
+        s->d_tris = nullptr;
+        s->d_mats = nullptr;
+        s->d_nodes = nullptr;
+        s->d_lights = nullptr;
+        s->d_spheres = nullptr;
+        s->d_snodes = nullptr;
+        s->d_ptri_id = nullptr;
+    }
     // d_ptris lies inside d_w4nodes' allocation unless the two are separate
     void* ptris = s->tri_off == kSeparateArrays ? (void*)s->d_ptris : nullptr;
     for (void* p : {(void*)s->d_tris, (void*)s->d_mats, (void*)s->d_nodes, (void*)s->d_lights,
@@ -504,36 +524,57 @@ int device_tree(rt_ctx* ctx, const rt_triangle* tris, uint32_t n, std::vector<rt
 
 namespace rtamd {
 
-uint64_t packed_record_bytes(const PackedTree& p, uint32_t wide) {
-    const uint64_t records = sizeof(PNode4) * ((uint64_t)p.w4nodes.size() + wide);
-    const uint64_t nb = (records + 255) / 256 * 256;
-    const uint64_t tb = sizeof(PTri) * (uint64_t)p.tris.size();
-    if (nb + tb >= (1ull << 32) || !nb || !tb) return records + tb;
+uint64_t packed_record_bytes(uint64_t records, uint64_t slots) {
+    const uint64_t rb = sizeof(PNode4) * records;
+    const uint64_t nb = (rb + 255) / 256 * 256;
+    const uint64_t tb = sizeof(PTri) * slots;
+    if (nb + tb >= (1ull << 32) || !nb || !tb) return rb + tb;
     return nb + tb;
 }
 
-void scene_drop_wide(PreparedScene& P) {
-    if (!P.wide) return;
-    P.bytes -= packed_record_bytes(P.packed, P.wide_records);
-    P.wide.reset();
-    P.wide_records = P.wide_need = 0;
-    P.bytes += packed_record_bytes(P.packed, 0);
-}
+namespace {
+// The arrays that stay as the caller gave them, with the sphere tree and the
+// triangles' ids, as parts of one allocation (scenes packed on the device).
+struct Arena {
+    size_t bytes = 0;
+    size_t tris, nodes, mats, lights, spheres, snodes, ids;
+    size_t take(size_t b) { const size_t o = bytes; bytes += (b + 255) / 256 * 256; return o; }
+    explicit Arena(const PreparedScene& P) {
+        const rt_scene_desc& d = P.desc;
+        tris = take(sizeof(rt_triangle) * (size_t)d.num_triangles);
+        nodes = take(sizeof(rt_bvh_node) * (size_t)d.num_nodes);
+        mats = take(sizeof(rt_material) * (size_t)d.num_materials);
+        lights = take(sizeof(rt_light) * (size_t)d.num_lights);
+        spheres = take(sizeof(rt_sphere) * (size_t)d.num_spheres);
+        snodes = take(P.sphere_tree ? sizeof(SphereNode) * P.snodes.size() : 0);
+        ids = take(sizeof(int32_t) * (size_t)P.leaf_slots);
+    }
+};
 
-int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& P) {
-    if (!ctx) return RT_ERR_INVALID;
-    if (!desc) return set_error(ctx, RT_ERR_INVALID, "rt_scene_upload: null argument");
-    // `user` keeps the caller's tree (the shader-order traversal walks it),
-    // `packsrc` is the tree the packed traversal is built from
-    rt_scene_desc user = *desc, packsrc = *desc;
-    P.tree_built = ctx->tuning.tree == RT_TREE_DEVICE;
+// What check_scene tests of the small arrays; a failure is left for it to name.
+bool small_arrays_ok(const rt_scene_desc& d) {
+    if (!d.num_materials || !d.materials || (d.num_lights && !d.lights) || (d.num_spheres && !d.spheres)) return false;
+    for (uint32_t i = 0; i < d.num_materials; ++i)
+        if (d.materials[i].type > 3u) return false;
+    for (uint32_t i = 0; i < d.num_lights; ++i)
+        if (d.lights[i].triangleIndex >= d.num_triangles) return false;
+    for (uint32_t i = 0; i < d.num_spheres; ++i)
+        if (d.spheres[i].materialIndex >= d.num_materials) return false;
+    return true;
+}
+}  // namespace
+
+namespace {
+// The host's half: validates and packs with one thread.  `packsrc` is the
+// tree to pack, `user` the caller's.
+int host_prepare(rt_ctx* ctx, rt_scene_desc& user, rt_scene_desc& packsrc, PreparedScene& P, bool plain) {
     if (P.tree_built) {
         RT_HIP(ctx, hipSetDevice(ctx->device));
-        int rc = device_tree(ctx, desc->triangles, desc->num_triangles, P.built);
+        int rc = device_tree(ctx, user.triangles, user.num_triangles, P.built);
         if (rc) return rc;
         packsrc.nodes = P.built.data();
         packsrc.num_nodes = (uint32_t)P.built.size();
-        if (!desc->nodes || desc->num_nodes == 0) user = packsrc;
+        if (!user.nodes || user.num_nodes == 0) user = packsrc;
     }
     SceneCheck pchk;
     try {
@@ -553,9 +594,33 @@ int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& P) {
         }
         if (P.packed.height > kMaxPackedHeight) P.fast = false;
     }
-    if (P.fast) {
+    P.given_records = (uint32_t)P.packed.w4nodes.size();
+    P.leaf_slots = (uint32_t)P.packed.tris.size();
+    if (P.fast && !plain) {
         RT_HIP(ctx, hipSetDevice(ctx->device));
         const int rc = wide_build(ctx, P.packed, nullptr, P.wide, P.wide_records, P.wide_need);
+        if (rc) return rc;
+    }
+    return RT_OK;
+}
+}  // namespace
+
+int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& P, bool plain) {
+    if (!ctx) return RT_ERR_INVALID;
+    if (!desc) return set_error(ctx, RT_ERR_INVALID, "rt_scene_upload: null argument");
+    // `user` keeps the caller's tree (the shader-order traversal walks it),
+    // `packsrc` is the tree the packed traversal is built from
+    rt_scene_desc user = *desc, packsrc = *desc;
+    P.tree_built = ctx->tuning.tree == RT_TREE_DEVICE;
+    const bool wide_layout = resolved_layout(ctx) == RT_LAYOUT_W4;
+    if (!plain && !P.tree_built && wide_layout && small_arrays_ok(*desc)) {
+        RT_HIP(ctx, hipSetDevice(ctx->device));
+        bool done = false;
+        const int rc = device_pack(ctx, *desc, P, &done);
+        if (rc) return rc;
+    }
+    if (!P.device_packed) {
+        const int rc = host_prepare(ctx, user, packsrc, P, plain);
         if (rc) return rc;
     }
     P.desc = user;
@@ -575,13 +640,55 @@ int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& P) {
                  sizeof(rt_sphere) * (uint64_t)user.num_spheres;
     if (P.sphere_tree) b += sizeof(SphereNode) * (uint64_t)P.snodes.size();
     if (P.fast) {
-        b += packed_record_bytes(P.packed, P.wide_records) + sizeof(int32_t) * (uint64_t)P.packed.tri_id.size();
+        b += sizeof(int32_t) * (uint64_t)P.leaf_slots;
+        b += packed_record_bytes((uint64_t)P.given_records + P.wide_records, P.leaf_slots);
         if (P.with_pnodes) b += sizeof(PNode) * (uint64_t)P.packed.nodes.size();
         if (P.with_qnodes) b += sizeof(PNodeQ) * (uint64_t)P.packed.qnodes.size();
     }
     P.bytes = b;
     return RT_OK;
 }
+
+namespace {
+// A scene packed on the device: its arrays in one allocation, the caller's
+// copied from the upload's scratch, then the records and triangles.
+int upload_packed(rt_ctx* ctx, rt_scene* s, const PreparedScene& P, uint64_t& bytes) {
+    const rt_scene_desc& d = P.desc;
+    const Arena A(P);
+    RT_HIP(ctx, hipMalloc((void**)&s->d_base, A.bytes));
+    char* b = s->d_base;
+    s->d_tris = (rt_triangle*)(b + A.tris);
+    s->d_nodes = (rt_bvh_node*)(b + A.nodes);
+    s->d_mats = (rt_material*)(b + A.mats);
+    if (d.num_lights) s->d_lights = (rt_light*)(b + A.lights);
+    if (d.num_spheres) s->d_spheres = (rt_sphere*)(b + A.spheres);
+    if (P.sphere_tree) s->d_snodes = (SphereNode*)(b + A.snodes);
+    s->d_ptri_id = (int32_t*)(b + A.ids);
+    s->wide = true;
+    const auto copy = [&](void* dst, const void* src, size_t n, hipMemcpyKind k) {
+        return n ? hipMemcpyAsync(dst, src, n, k, nullptr) : hipSuccess;
+    };
+    RT_HIP(ctx, copy(s->d_tris, wide_triangles(*P.wide), sizeof(rt_triangle) * (size_t)d.num_triangles, hipMemcpyDeviceToDevice));
+    RT_HIP(ctx, copy(s->d_nodes, wide_nodes(*P.wide), sizeof(rt_bvh_node) * (size_t)d.num_nodes, hipMemcpyDeviceToDevice));
+    RT_HIP(ctx, copy(s->d_mats, d.materials, sizeof(rt_material) * (size_t)d.num_materials, hipMemcpyHostToDevice));
+    RT_HIP(ctx, copy(s->d_lights, d.lights, sizeof(rt_light) * (size_t)d.num_lights, hipMemcpyHostToDevice));
+    RT_HIP(ctx, copy(s->d_spheres, d.spheres, sizeof(rt_sphere) * (size_t)d.num_spheres, hipMemcpyHostToDevice));
+    if (P.sphere_tree)
+        RT_HIP(ctx, copy(s->d_snodes, P.snodes.data(), sizeof(SphereNode) * P.snodes.size(), hipMemcpyHostToDevice));
+    // (the arrays' own bytes, as for separate allocations)
+    bytes += sizeof(rt_triangle) * (uint64_t)d.num_triangles + sizeof(rt_material) * (uint64_t)d.num_materials +
+             sizeof(rt_bvh_node) * (uint64_t)d.num_nodes + sizeof(rt_light) * (uint64_t)d.num_lights +
+             sizeof(rt_sphere) * (uint64_t)d.num_spheres + sizeof(int32_t) * (uint64_t)P.leaf_slots;
+    if (P.sphere_tree) bytes += sizeof(SphereNode) * (uint64_t)P.snodes.size();
+    int rc = alloc_records(ctx, s, (size_t)P.given_records + P.wide_records, P.leaf_slots, bytes);
+    if (rc) return rc;
+    rc = wide_emit(ctx, *P.wide, P.wide_records, s->d_w4nodes, s->d_ptris, s->d_ptri_id, nullptr);
+    if (rc) return rc;
+    // the caller's arrays are free, and any stream may trace, once the upload returns
+    RT_HIP(ctx, hipStreamSynchronize(nullptr));
+    return RT_OK;
+}
+}  // namespace
 
 int scene_commit(rt_ctx* ctx, PreparedScene& P, rt_scene** out) {
     if (!ctx || !out) return RT_ERR_INVALID;
@@ -595,6 +702,10 @@ int scene_commit(rt_ctx* ctx, PreparedScene& P, rt_scene** out) {
     uint64_t bytes = 0;
     int rc = RT_OK;
     do {
+        if (P.device_packed) {
+            rc = upload_packed(ctx, s, P, bytes);
+            break;
+        }
         if ((rc = upload_array(ctx, &s->d_tris, desc->triangles, desc->num_triangles, bytes))) break;
         if ((rc = upload_array(ctx, &s->d_mats, desc->materials, desc->num_materials, bytes))) break;
         if ((rc = upload_array(ctx, &s->d_nodes, desc->nodes, desc->num_nodes, bytes))) break;
@@ -618,7 +729,7 @@ int scene_commit(rt_ctx* ctx, PreparedScene& P, rt_scene** out) {
     }
     s->root_ref = fast ? packed.root : kEmptyRoot;
     s->frame = packed.frame;
-    s->root4 = !fast ? kEmptyRoot : s->wide ? (int32_t)packed.w4nodes.size() : packed.root4;
+    s->root4 = !fast ? kEmptyRoot : s->wide ? (int32_t)P.given_records : packed.root4;
     s->stack4 = fast ? std::max(packed.stack4, P.wide_need) : 0;
     P.wide.reset();
     s->packed_height = fast ? packed.height : 0;

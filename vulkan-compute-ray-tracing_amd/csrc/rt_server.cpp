@@ -440,11 +440,12 @@ extern "C" int rt_server_destroy(rt_server* S) {
 
 extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint64_t* scene_id) {
     if (!S || !desc || !scene_id) return RT_ERR_INVALID;
-    // the host half first: validated and packed, so the scene's device bytes
-    // are known before anything is allocated on the device
+    // validated and packed first, in scratch, so the scene's device bytes are
+    // known before any of them is allocated
+    // (one upload at a time: its scratch is the context's)
+    std::lock_guard<std::mutex> up(S->upload_mu);
     PreparedScene prep;
     {
-        std::lock_guard<std::mutex> up(S->upload_mu);
         int rc = scene_prepare(S->ctx, desc, prep);
         if (rc) return fail(S, rc, std::string("rt_server_scene_add: ") + rt_last_error(S->ctx));
         if (!prep.fast) return fail(S, RT_ERR_UNSUPPORTED, "rt_server_scene_add: scene without the packed traversal");
@@ -482,7 +483,6 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
             S->st.scenes_refused++;
         }
     }
-    std::lock_guard<std::mutex> up(S->upload_mu);
     for (rt_scene* e : evicted) rt_scene_release(S->ctx, e);      // freed before the new scene is allocated
     evicted.clear();
     if (!admitted) return fail(S, RT_ERR_NOMEM, "rt_server_scene_add: HBM budget exceeded by scenes with pending work");
@@ -494,10 +494,16 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || (uint64_t)free_b >= bytes + margin) break;
         // the traversal tree and its scratch go before any resident scene
         if (prep.wide) {
-            scene_drop_wide(prep);
+            prep = PreparedScene{};
+            const int rc = scene_prepare(S->ctx, desc, prep, true);
             std::lock_guard<std::mutex> lk(S->mu);
-            S->resident -= bytes - prep.bytes;
-            bytes = prep.bytes;
+            S->resident -= bytes;
+            bytes = rc ? 0 : prep.bytes;
+            S->resident += bytes;
+            if (rc) {
+                S->st.scenes_refused++;
+                return fail(S, rc, std::string("rt_server_scene_add: ") + rt_last_error(S->ctx));
+            }
             continue;
         }
         uint64_t v = 0;

@@ -73,6 +73,24 @@ __device__ inline double wave_sum(double v) {
     return v;
 }
 
+// Adds every thread's v to *total, one atomic a block.  Called by whole blocks of 256.
+__device__ inline void block_add(double v, double* total) {
+    __shared__ double part[4];
+    v = wave_sum(v);
+    if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const double sum = (part[0] + part[1]) + (part[2] + part[3]);
+        if (sum != 0.0) atomicAdd(total, sum);
+    }
+}
+
+// Morton code of a box's centre, 16 bits an axis.
+__device__ __forceinline__ uint64_t wide_key(uint4 w) {
+    return (spread3(((w.x & 0xffffu) + (w.x >> 16)) >> 1) << 2) | (spread3(((w.y & 0xffffu) + (w.y >> 16)) >> 1) << 1) |
+           spread3(((w.z & 0xffffu) + (w.z >> 16)) >> 1);
+}
+
 // One thread per child slot of the caller's records: the words and code of
 // each leaf, and the summed area of the inner children (the records a ray
 // reads, by the surface-area measure).
@@ -93,12 +111,10 @@ __global__ __launch_bounds__(256) void k_wide_leaves(const PNode4* __restrict__ 
         }
         const uint32_t leaf = (uint32_t)~ref;
         words[leaf] = make_uint4(x, y, z, 0u);
-        keys[leaf] = (spread3(((x & 0xffffu) + (x >> 16)) >> 1) << 2) |
-                     (spread3(((y & 0xffffu) + (y >> 16)) >> 1) << 1) | spread3(((z & 0xffffu) + (z >> 16)) >> 1);
+        keys[leaf] = wide_key(words[leaf]);
         vals[leaf] = leaf;
     }
-    sum = wave_sum(sum);
-    if ((threadIdx.x & 63u) == 0 && sum != 0.0) atomicAdd(cost, sum);
+    block_add(sum, cost);
 }
 
 // Leaf words in sorted order.
@@ -181,14 +197,17 @@ struct WideRec {
     uint32_t rank[4];            // preorder rank of an internal child
 };
 
-__global__ void k_wide_root(WideRec* recs, uint32_t* level_count, uint32_t* need, double* cost) {
+// The first level of the collapse, and its sums at zero (cost[1], the caller's
+// tree's, only with zero_given).
+__global__ void k_wide_root(WideRec* recs, uint32_t* level_count, uint32_t* need, double* cost, uint32_t zero_given) {
     const uint32_t t = threadIdx.x;
     if (t < kMaxLevels + 1) level_count[t] = t == 0 ? 1u : 0u;
     if (t == 0) {
         recs[0].node = 0;
         recs[0].lo = recs[0].left = recs[0].need = 0u;
         *need = 0u;
-        cost[0] = cost[1] = 0.0;
+        cost[0] = 0.0;
+        if (zero_given) cost[1] = 0.0;
     }
 }
 
@@ -274,8 +293,7 @@ __global__ __launch_bounds__(256) void k_wide_collapse(const int2* __restrict__ 
             }
         }
     }
-    sum = wave_sum(sum);
-    if ((threadIdx.x & 63u) == 0 && sum != 0.0) atomicAdd(cost, sum);
+    block_add(sum, cost);
 }
 
 // The records, numbered from `first` in preorder; leaf refs are ~(sorted position).
@@ -324,24 +342,168 @@ __global__ __launch_bounds__(256) void k_wide_place(const PNode4* __restrict__ g
 
 }  // namespace
 
-// What a build keeps between its two halves, in one device allocation.
-struct WideScratch {
-    char* base = nullptr;
-    ~WideScratch() { if (base) (void)hipFree(base); }
+// Where a build's arrays lie in its one device allocation: what packing makes
+// for it, then what is only used by the build (from `overlay` on).
+struct WideLayout {
+    size_t bytes = 0, overlay = 0;
+    size_t raw_tris = 0, raw_nodes = 0;
+    size_t given = 0, tris = 0, ids = 0, words = 0, keys = 0, vals = 0, counts = 0, cost = 0, facts = 0;
+    size_t sorted = 0, keys2 = 0, order = 0, kids = 0, far = 0, boxes = 0, recs = 0, rank = 0, tmp = 0;
+    size_t lvl[kPyramidLevels] = {};
+    size_t sort_bytes = 0, scan_bytes = 0;
+    size_t take(size_t b) { const size_t o = bytes; bytes += align256(b); return o; }
+    // n leaves and `records` of the caller's records, at most
+    int wide(rt_ctx* ctx, uint32_t n, uint32_t records, hipStream_t s) {
+        RT_HIP(ctx, rocprim::radix_sort_pairs(nullptr, sort_bytes, (uint64_t*)nullptr, (uint64_t*)nullptr,
+                                              (uint32_t*)nullptr, (uint32_t*)nullptr, n, 0u, kCodeBits, s));
+        RT_HIP(ctx, rocprim::exclusive_scan(nullptr, scan_bytes, (uint32_t*)nullptr, (uint32_t*)nullptr, 0u, n,
+                                            rocprim::plus<uint32_t>(), s));
+        given = take(sizeof(PNode4) * (size_t)records);
+        tris = take(sizeof(PTri) * (size_t)n);
+        ids = take(4 * (size_t)n);
+        words = take(16 * (size_t)n);
+        keys = take(8 * (size_t)n);
+        vals = take(4 * (size_t)n);
+        counts = take(4 * (kMaxLevels + 2));
+        cost = take(16);
+        facts = take(64);
+        overlay = bytes;
+        sorted = take(16 * (size_t)n);
+        keys2 = take(8 * (size_t)n);
+        order = take(4 * (size_t)n);
+        kids = take(8 * (size_t)n);
+        far = take(4 * (size_t)n);
+        boxes = take(16 * (size_t)n);
+        recs = take(sizeof(WideRec) * (size_t)std::max(1u, n / 2u));
+        rank = take(4 * (size_t)n);
+        uint32_t count = n;
+        for (int k = 1; k < kPyramidLevels; ++k) {
+            count = (count + 63u) / 64u;
+            lvl[k] = take(16 * (size_t)count);
+        }
+        tmp = take(std::max(sort_bytes, scan_bytes));
+        return RT_OK;
+    }
 };
 
+// A build between its two halves.  Its memory is the context's upload
+// workspace where that is small, else an allocation of its own.
 struct WideTree {
-    WideScratch mem;
+    char* base = nullptr;
+    bool own = false;
     PNode4* given = nullptr;
     PTri* tris = nullptr;
     int32_t* ids = nullptr;
-    uint4 *sorted = nullptr, *boxes = nullptr;
-    uint32_t *order = nullptr, *rank_to_index = nullptr, *place = nullptr;
+    uint4 *words = nullptr, *sorted = nullptr, *boxes = nullptr;
+    uint64_t* keys = nullptr;
+    uint32_t *vals = nullptr, *order = nullptr, *rank_to_index = nullptr, *place = nullptr;
     WideRec* recs = nullptr;
     uint32_t n = 0, n_given = 0;
+    const rt_triangle* raw_tris = nullptr;    // the caller's arrays, when packed on the device
+    const rt_bvh_node* raw_nodes = nullptr;
+    ~WideTree() { if (own && base) (void)hipFree(base); }
+    // false: no room
+    bool allocate(rt_ctx* ctx, size_t bytes) {
+        if (bytes <= kUploadKept) {
+            if (ensure_workspace(ctx, kWsUpload, bytes) == RT_OK) {
+                base = (char*)ctx->ws[kWsUpload];
+                return true;
+            }
+        } else if (hipMalloc((void**)&base, bytes) == hipSuccess) {
+            own = true;
+            return true;
+        }
+        (void)hipGetLastError();
+        base = nullptr;
+        return false;
+    }
+    void bind(const WideLayout& L, uint32_t leaves, uint32_t records) {
+        n = leaves;
+        n_given = records;
+        given = (PNode4*)(base + L.given);
+        tris = (PTri*)(base + L.tris);
+        ids = (int32_t*)(base + L.ids);
+        words = (uint4*)(base + L.words);
+        keys = (uint64_t*)(base + L.keys);
+        vals = (uint32_t*)(base + L.vals);
+        sorted = (uint4*)(base + L.sorted);
+        boxes = (uint4*)(base + L.boxes);
+        order = (uint32_t*)(base + L.order);
+        rank_to_index = (uint32_t*)(base + L.rank);
+        place = vals;                              // the sort's input indices, free by then
+        recs = (WideRec*)(base + L.recs);
+    }
 };
 
 void WideTreeDelete::operator()(WideTree* t) const { delete t; }
+
+// The tree over t's leaves (words, keys, vals, and the caller's cost in
+// cost[1] are set).  *better stays false where the caller's tree is to be
+// traversed as it is.  Waits for the build.
+static int wide_core(rt_ctx* ctx, WideTree& t, const WideLayout& L, const QFrame& f, hipStream_t s, uint32_t& records,
+                     uint32_t& need, bool* better) {
+    const uint32_t n = t.n;
+    const uint32_t cap = std::max(1u, n / 2u);
+    char* b = t.base;
+    uint64_t* keys2 = (uint64_t*)(b + L.keys2);
+    int2* kids = (int2*)(b + L.kids);
+    uint32_t *far = (uint32_t*)(b + L.far), *counts = (uint32_t*)(b + L.counts);
+    uint32_t* flags = (uint32_t*)t.words;         // the unsorted words are done when the collapse starts
+    uint32_t* d_need = counts + kMaxLevels + 1;
+    double* cost = (double*)(b + L.cost);
+    WPyramid pyr{};
+    pyr.count[0] = n;
+    pyr.levels = 1;
+    while (pyr.levels < (uint32_t)kPyramidLevels && pyr.count[pyr.levels - 1] > 1) {
+        pyr.count[pyr.levels] = (pyr.count[pyr.levels - 1] + 63u) / 64u;
+        ++pyr.levels;
+    }
+    auto grid = [&](uint64_t work) {
+        return dim3((uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((work + 255) / 256, (uint64_t)ctx->num_cus * 16u)));
+    };
+    const dim3 block(256);
+    size_t sort_bytes = L.sort_bytes, scan_bytes = L.scan_bytes;
+    RT_HIP(ctx, rocprim::radix_sort_pairs((void*)(b + L.tmp), sort_bytes, t.keys, keys2, t.vals, t.order, n, 0u, kCodeBits, s));
+    hipLaunchKernelGGL(k_wide_sorted, grid(n), block, 0, s, t.words, t.order, n, t.sorted);
+    hipLaunchKernelGGL(k_wide_tree, grid(n - 1), block, 0, s, keys2, n, kids, far);
+    pyr.lvl[0] = t.sorted;
+    for (uint32_t k = 1; k < pyr.levels; ++k) pyr.lvl[k] = (uint4*)(b + L.lvl[k]);
+    for (uint32_t k = 0; k + 1 < pyr.levels; ++k)
+        hipLaunchKernelGGL(k_wide_pyramid, grid((uint64_t)pyr.count[k + 1] * 64u), block, 0, s, pyr, k,
+                           (uint4*)(b + L.lvl[k + 1]));
+    hipLaunchKernelGGL(k_wide_boxes, grid(n - 1), block, 0, s, pyr, n, far, t.boxes);
+    RT_HIP(ctx, hipGetLastError());
+    int rc = launch_fill_u32(ctx, flags, 0u, n, s);
+    if (rc) return rc;
+    // levels until one is empty; their sizes live on the device and are read
+    // back every kLevelsPerSync levels
+    uint32_t h[kMaxLevels + 2] = {};
+    double c[2] = {0.0, 0.0};
+    uint32_t level = 0;
+    for (;;) {
+        const uint32_t end = std::min(level + kLevelsPerSync, kMaxLevels);
+        for (; level < end; ++level)
+            hipLaunchKernelGGL(k_wide_collapse, grid(cap), block, 0, s, kids, far, t.boxes, f, level, cap, t.recs, counts,
+                               flags, d_need, cost);
+        RT_HIP(ctx, hipGetLastError());
+        RT_HIP(ctx, hipMemcpyAsync(h, counts, sizeof h, hipMemcpyDeviceToHost, s));
+        RT_HIP(ctx, hipMemcpyAsync(c, cost, sizeof c, hipMemcpyDeviceToHost, s));
+        RT_HIP(ctx, hipStreamSynchronize(s));
+        if (h[level] == 0 || level == kMaxLevels) break;
+    }
+    if (h[level] != 0) return RT_OK;              // deeper than kMaxLevels levels
+    uint64_t R = 0;
+    for (uint32_t l = 0; l < level; ++l) R += h[l];
+    // more records than reserved, a stack no kernel variant holds, or a
+    // caller's tree that is the better one (its boxes' summed area smaller)
+    if (R > cap || h[kMaxLevels + 1] + 1u > kMaxWideStack || !(c[0] < c[1])) return RT_OK;
+    RT_HIP(ctx, rocprim::exclusive_scan((void*)(b + L.tmp), scan_bytes, flags, t.rank_to_index, 0u, n,
+                                        rocprim::plus<uint32_t>(), s));
+    records = (uint32_t)R;
+    need = h[kMaxLevels + 1] + 1u;
+    *better = true;
+    return RT_OK;
+}
 
 int wide_build(rt_ctx* ctx, const PackedTree& packed, hipStream_t s, std::unique_ptr<WideTree, WideTreeDelete>& out,
                uint32_t& records, uint32_t& need) {
@@ -351,108 +513,27 @@ int wide_build(rt_ctx* ctx, const PackedTree& packed, hipStream_t s, std::unique
     if (n < 2 || G == 0 || packed.root4 != 0) return RT_OK;
     std::unique_ptr<WideTree, WideTreeDelete> t(new (std::nothrow) WideTree());
     if (!t) return RT_OK;
-    t->n = n;
-    t->n_given = G;
-    const uint32_t cap = std::max(1u, n / 2u);
-    size_t sort_bytes = 0, scan_bytes = 0;
-    RT_HIP(ctx, rocprim::radix_sort_pairs(nullptr, sort_bytes, (uint64_t*)nullptr, (uint64_t*)nullptr,
-                                          (uint32_t*)nullptr, (uint32_t*)nullptr, n, 0u, kCodeBits, s));
-    RT_HIP(ctx, rocprim::exclusive_scan(nullptr, scan_bytes, (uint32_t*)nullptr, (uint32_t*)nullptr, 0u, n,
-                                        rocprim::plus<uint32_t>(), s));
-    WPyramid pyr{};
-    pyr.count[0] = n;
-    pyr.levels = 1;
-    while (pyr.levels < (uint32_t)kPyramidLevels && pyr.count[pyr.levels - 1] > 1) {
-        pyr.count[pyr.levels] = (pyr.count[pyr.levels - 1] + 63u) / 64u;
-        ++pyr.levels;
-    }
-    size_t off = 0;
-    auto take = [&](size_t bytes) { const size_t o = off; off += align256(bytes); return o; };
-    const size_t o_given = take(sizeof(PNode4) * (size_t)G), o_tris = take(sizeof(PTri) * (size_t)n);
-    const size_t o_ids = take(4 * (size_t)n), o_words = take(16 * (size_t)n), o_sorted = take(16 * (size_t)n);
-    const size_t o_keys = take(8 * (size_t)n), o_keys2 = take(8 * (size_t)n);
-    const size_t o_vals = take(4 * (size_t)n), o_order = take(4 * (size_t)n);
-    const size_t o_kids = take(8 * (size_t)n), o_far = take(4 * (size_t)n), o_boxes = take(16 * (size_t)n);
-    const size_t o_recs = take(sizeof(WideRec) * (size_t)cap);
-    const size_t o_rank = take(4 * (size_t)n), o_counts = take(4 * (kMaxLevels + 2)), o_cost = take(16);
-    const size_t o_tmp = take(std::max(sort_bytes, scan_bytes));
-    size_t o_lvl[kPyramidLevels] = {};
-    for (uint32_t L = 1; L < pyr.levels; ++L) o_lvl[L] = take(16 * (size_t)pyr.count[L]);
+    WideLayout L;
+    int rc = L.wide(ctx, n, G, s);
+    if (rc) return rc;
     // no room for the scratch: the caller's tree is traversed as it is
-    if (hipMalloc((void**)&t->mem.base, off) != hipSuccess) {
-        (void)hipGetLastError();
-        t->mem.base = nullptr;
-        return RT_OK;
-    }
-    char* b = t->mem.base;
-    t->given = (PNode4*)(b + o_given);
-    t->tris = (PTri*)(b + o_tris);
-    t->ids = (int32_t*)(b + o_ids);
-    t->sorted = (uint4*)(b + o_sorted);
-    t->boxes = (uint4*)(b + o_boxes);
-    t->order = (uint32_t*)(b + o_order);
-    t->rank_to_index = (uint32_t*)(b + o_rank);
-    t->place = (uint32_t*)(b + o_vals);           // the sort's input indices, free by then
-    t->recs = (WideRec*)(b + o_recs);
-    uint4* words = (uint4*)(b + o_words);
-    uint64_t *keys = (uint64_t*)(b + o_keys), *keys2 = (uint64_t*)(b + o_keys2);
-    uint32_t* vals = (uint32_t*)(b + o_vals);
-    int2* kids = (int2*)(b + o_kids);
-    uint32_t *far = (uint32_t*)(b + o_far), *counts = (uint32_t*)(b + o_counts);
-    uint32_t* flags = (uint32_t*)words;           // the unsorted words are done when the collapse starts
-    uint32_t* d_need = counts + kMaxLevels + 1;
-    double* cost = (double*)(b + o_cost);
+    if (!t->allocate(ctx, L.bytes)) return RT_OK;
+    t->bind(L, n, G);
+    uint32_t* counts = (uint32_t*)(t->base + L.counts);
+    double* cost = (double*)(t->base + L.cost);
     RT_HIP(ctx, hipMemcpyAsync(t->given, packed.w4nodes.data(), sizeof(PNode4) * (size_t)G, hipMemcpyHostToDevice, s));
     RT_HIP(ctx, hipMemcpyAsync(t->tris, packed.tris.data(), sizeof(PTri) * (size_t)n, hipMemcpyHostToDevice, s));
     RT_HIP(ctx, hipMemcpyAsync(t->ids, packed.tri_id.data(), 4 * (size_t)n, hipMemcpyHostToDevice, s));
-    auto grid = [&](uint64_t work) {
-        return dim3((uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((work + 255) / 256, (uint64_t)ctx->num_cus * 16u)));
-    };
     const dim3 block(256);
-    const QFrame& f = packed.frame;
-    hipLaunchKernelGGL(k_wide_root, dim3(1), block, 0, s, t->recs, counts, d_need, cost);
-    hipLaunchKernelGGL(k_wide_leaves, grid(4ull * G), block, 0, s, t->given, G, f, words, keys, vals, cost + 1);
+    const dim3 grid((uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((4ull * G + 255) / 256, (uint64_t)ctx->num_cus * 8u)));
+    hipLaunchKernelGGL(k_wide_root, dim3(1), block, 0, s, t->recs, counts, counts + kMaxLevels + 1, cost,
+                       1u);
+    hipLaunchKernelGGL(k_wide_leaves, grid, block, 0, s, t->given, G, packed.frame, t->words, t->keys, t->vals, cost + 1);
     RT_HIP(ctx, hipGetLastError());
-    RT_HIP(ctx, rocprim::radix_sort_pairs((void*)(b + o_tmp), sort_bytes, keys, keys2, vals, t->order, n, 0u, kCodeBits, s));
-    hipLaunchKernelGGL(k_wide_sorted, grid(n), block, 0, s, words, t->order, n, t->sorted);
-    hipLaunchKernelGGL(k_wide_tree, grid(n - 1), block, 0, s, keys2, n, kids, far);
-    pyr.lvl[0] = t->sorted;
-    for (uint32_t L = 1; L < pyr.levels; ++L) pyr.lvl[L] = (uint4*)(b + o_lvl[L]);
-    for (uint32_t L = 0; L + 1 < pyr.levels; ++L)
-        hipLaunchKernelGGL(k_wide_pyramid, grid((uint64_t)pyr.count[L + 1] * 64u), block, 0, s, pyr, L,
-                           (uint4*)(b + o_lvl[L + 1]));
-    hipLaunchKernelGGL(k_wide_boxes, grid(n - 1), block, 0, s, pyr, n, far, t->boxes);
-    RT_HIP(ctx, hipGetLastError());
-    int rc = launch_fill_u32(ctx, flags, 0u, n, s);
+    bool better = false;
+    rc = wide_core(ctx, *t, L, packed.frame, s, records, need, &better);
     if (rc) return rc;
-    // levels until one is empty; their sizes live on the device and are read
-    // back every kLevelsPerSync levels
-    uint32_t h[kMaxLevels + 2] = {};
-    uint32_t level = 0;
-    for (;;) {
-        const uint32_t end = std::min(level + kLevelsPerSync, kMaxLevels);
-        for (; level < end; ++level)
-            hipLaunchKernelGGL(k_wide_collapse, grid(cap), block, 0, s, kids, far, t->boxes, f, level, cap, t->recs, counts,
-                               flags, d_need, cost);
-        RT_HIP(ctx, hipGetLastError());
-        RT_HIP(ctx, hipMemcpyAsync(h, counts, sizeof h, hipMemcpyDeviceToHost, s));
-        RT_HIP(ctx, hipStreamSynchronize(s));
-        if (h[level] == 0 || level == kMaxLevels) break;
-    }
-    if (h[level] != 0) return RT_OK;              // deeper than kMaxLevels levels
-    uint64_t R = 0;
-    for (uint32_t l = 0; l < level; ++l) R += h[l];
-    double c[2] = {0.0, 0.0};
-    RT_HIP(ctx, hipMemcpyAsync(c, cost, sizeof c, hipMemcpyDeviceToHost, s));
-    RT_HIP(ctx, rocprim::exclusive_scan((void*)(b + o_tmp), scan_bytes, flags, t->rank_to_index, 0u, n,
-                                        rocprim::plus<uint32_t>(), s));
-    RT_HIP(ctx, hipStreamSynchronize(s));
-    // more records than reserved, a stack no kernel variant holds, or a
-    // caller's tree that is the better one (its boxes' summed area smaller)
-    if (R > cap || h[kMaxLevels + 1] + 1u > kMaxWideStack || !(c[0] < c[1])) return RT_OK;
-    records = (uint32_t)R;
-    need = h[kMaxLevels + 1] + 1u;
-    out = std::move(t);
+    if (better) out = std::move(t);
     return RT_OK;
 }
 
@@ -468,5 +549,8 @@ int wide_emit(rt_ctx* ctx, const WideTree& t, uint32_t records, PNode4* nodes, P
     RT_HIP(ctx, hipGetLastError());
     return RT_OK;
 }
+
+const rt_triangle* wide_triangles(const WideTree& t) { return t.raw_tris; }
+const rt_bvh_node* wide_nodes(const WideTree& t) { return t.raw_nodes; }
 
 }  // namespace rtamd
