@@ -319,6 +319,8 @@ static_assert(kSegments == 1u << kSegmentShift, "segments are a power of two");
 constexpr uint32_t kCursorStride = 32;
 constexpr uint32_t kChunkRays = 64;             // rays a wave takes from a cursor at once,
 constexpr uint32_t kChunkedRays = 192;          // where there are this many for each wave
+constexpr uint32_t kFitRun = 2;                 // rays in a row that a wave takes where every wave
+constexpr uint32_t kDealRun = 8;                // gets its rays at the start, and from the cursors
 constexpr uint32_t kCursorBlock = kSegments * kCursorStride;
 constexpr uint32_t kCursorBlocks = 256;
 // A render's per-bounce counters (rt_ctx::d_counters): [b] = live rays entering bounce b.

@@ -225,6 +225,7 @@ struct TraceIo {
     uint32_t steal;           // idle lanes that make a drained wave share work (65: never)
     uint32_t simds;           // SIMDs of the device (plan_launch)
     unsigned long long* sums; // counting variant: totals of node and triangle records, or null
+    uint32_t deal;            // waves fetching from the cursors may take runs from all over the launch
 };
 
 __device__ __forceinline__ float lo16(uint32_t w) { return (float)(w & 0xffffu); }
@@ -349,6 +350,21 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
     uint32_t c_next = 0, c_end = 0;
     bool used_up = false;           // nothing is left past c_end
     const bool chunked = !io.order && n >= plan.blocks * (BLOCK / 64) * kChunkedRays;
+    // Neighbouring rays of a camera meet the same silhouette, so 64 of them in
+    // one wave are often 64 long rays, and the launch waits for that wave long
+    // after the others have ended.  Where a launch has few rays for each wave,
+    // waves therefore take runs of a few rays from all over the launch instead
+    // of 64 in a row: kFitRun where every wave gets its rays at the start
+    // (longer runs even out less), kDealRun in a query whose waves fetch rays
+    // as they go (runs of two cost clusters nothing but a soup 10%).  us a
+    // query: camera rays on an 81,920-triangle icosphere 100,000 90 -> 64,
+    // 300,000 122 -> 97, 524,288 149 -> 133; on 262,144-triangle clusters
+    // 65,536 100 -> 74, 524,288 212 -> 198.  Rays without order pay for the
+    // scattered reads: 0 to 2% (65,536 on 1,024 triangles 44.0 -> 46.7).  Not
+    // where waves take whole chunks (a 4k frame is the same either way: there
+    // are enough rays to even the waves out), and not in a render's bounces
+    // that use the cursors (four 960x540 frames 1,200 -> 1,240).
+    const uint32_t deal = !BATCHED && io.deal && !fits && !chunked && !io.order ? n / 64u * kDealRun : 0u;
     uint32_t ray_i = 0;
     RayIn r{};
     f3 bo{0.0f, 0.0f, 0.0f};        // ray origin in the box frame
@@ -603,17 +619,21 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
         if (!drained && n_idle >= io.refill) {
             // the rays left over, then new ones
             const uint32_t old_lo = c_next, old_n = c_end - c_next;
-            uint32_t new_n = 0, c_first = 0;
+            uint32_t new_n = 0, c_first = 0, fit_ray = n;
             c_next = old_lo + min(old_n, n_idle);
             if (n_idle > old_n && !used_up) {
                 if (fits) {
-                    // one run of rays to the blocks of each XCD
+                    // the rays of each XCD's blocks are neighbours
                     const uint32_t b = plan.blocks % kXcds == 0
                                            ? (blockIdx.x % kXcds) * (plan.blocks / kXcds) + blockIdx.x / kXcds : blockIdx.x;
-                    const uint64_t first =
-                        (uint64_t)(b * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(tid / 64u)) * plan.per_wave;
-                    c_first = (uint32_t)(first < n ? first : n);
-                    c_end = n - c_first > plan.per_wave ? c_first + plan.per_wave : n;
+                    const uint32_t waves = plan.blocks * (BLOCK / 64);
+                    const uint32_t wave = b * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(tid / 64u);
+                    // runs of `run` rays, one from each row of waves * run
+                    // rays; the last row's are shorter if per_wave is odd
+                    const uint32_t run = BATCHED || io.order ? plan.per_wave : min(kFitRun, plan.per_wave);
+                    const uint32_t row = lane / run;
+                    const uint32_t len = min(run, plan.per_wave - min(row * run, plan.per_wave));
+                    if (lane < plan.per_wave) fit_ray = row * run * waves + wave * len + (lane - row * run);
                     used_up = true;
                 } else {
                     const uint32_t take = chunked ? kChunkRays : n_idle - old_n;
@@ -640,6 +660,10 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
             uint32_t mine = n;
             if (rank < old_n) mine = old_lo + rank;
             else if (rank - old_n < new_n) mine = c_first + (rank - old_n);
+            if (fits) mine = fit_ray;
+            // 64 positions in a row are a run from each of 64 / kDealRun rows
+            if (mine < deal * (64u / kDealRun))
+                mine = mine / kDealRun % (64u / kDealRun) * deal + mine / 64u * kDealRun + mine % kDealRun;
             if (used_up && c_next == c_end) {
                 drained = true;
                 // a drained wave holds the launch's tail: it issues ahead of
