@@ -425,9 +425,22 @@ int launch_fill_u32(rt_ctx* ctx, uint32_t* p, uint32_t value, uint32_t count, hi
 
 // Batched traversal from caller-filled device tables (rt_batch.hip): the
 // server's per-slot launches.  stack_need = the scenes' largest stack4;
-// `cursor` holds kCursorBlock words (reset by the launch).
+// `cursor` holds kCursorBlock words, their segment words zero.
 int launch_batch_dynamic(rt_ctx* ctx, const BatchIo& bio, uint32_t* cursor, uint32_t total, uint32_t stack_need,
                          uint32_t refill, hipStream_t s);
+// A request's rays and hits in host memory as the device addresses them, in
+// 8-byte words; null where they are copied by other means.
+struct HostSpan {
+    const uint64_t* rays;
+    uint64_t* hits;
+};
+// Before a batch: the requests' rays to the device, and the segment words of
+// `cursor` to zero.
+int launch_gather(rt_ctx* ctx, const BatchIo& bio, const HostSpan* d_spans, rt_ray* d_rays, uint32_t total,
+                  uint32_t* cursor, hipStream_t s);
+// After it: its hits to the requests' buffers.
+int launch_scatter(rt_ctx* ctx, const BatchIo& bio, const HostSpan* d_spans, const rt_hit* d_hits, uint32_t total,
+                   hipStream_t s);
 
 // A scene is a device resource: any context on its device may trace it.
 inline bool scene_usable(const rt_ctx* c, const rt_scene* s);

@@ -53,7 +53,8 @@ struct Request {
     bool done = false;
     bool detached = false;       // nobody waits: freed on completion
     bool running = false;        // taken by a slot
-    bool direct = false;         // caller buffers are page-locked: DMA in place
+    bool direct = false;         // caller buffers are page-locked: used in place
+    HostSpan span{};             // direct: the buffers as kernels address them, or null
     uint32_t offset = 0;         // first ray in the slot's staging
 };
 
@@ -67,6 +68,26 @@ bool pinned(const void* p) {
     return a.type == hipMemoryTypeHost;
 }
 
+// The device's address of the page-locked host buffer [p, p + bytes), or null
+// where kernels cannot have all of it in 8-byte words.
+uint64_t* mapped(const void* p, size_t bytes) {
+    hipPointerAttribute_t a;
+    uintptr_t base = 0;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeHost || !a.devicePointer ||
+        ((uintptr_t)a.devicePointer & 7u) ||
+        hipPointerGetAttribute(&base, HIP_POINTER_ATTRIBUTE_RANGE_START_ADDR, (hipDeviceptr_t)a.devicePointer) !=
+            hipSuccess ||
+        hipPointerGetAttribute(&size, HIP_POINTER_ATTRIBUTE_RANGE_SIZE, (hipDeviceptr_t)a.devicePointer) !=
+            hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    const uintptr_t at = (uintptr_t)a.devicePointer;
+    if (at < base || at - base > size || size - (at - base) < bytes) return nullptr;
+    return (uint64_t*)a.devicePointer;
+}
+
 struct Slot {
     rt_ctx* ctx = nullptr;
     hipStream_t stream = nullptr;
@@ -75,12 +96,10 @@ struct Slot {
     rt_hit* d_hits = nullptr;
     rt_ray* h_rays = nullptr;
     rt_hit* h_hits = nullptr;
-    BatchEntry* d_table = nullptr;
-    BatchEntry* h_table = nullptr;
-    uint32_t* d_offsets = nullptr;
-    uint32_t* h_offsets = nullptr;
-    uint32_t* d_chunk = nullptr;
-    uint32_t* h_chunk = nullptr;
+    uint64_t* d_tables = nullptr;        // a batch's tables, packed (Tables)
+    uint64_t* h_tables = nullptr;
+    uint64_t* m_rays = nullptr;          // h_rays and h_hits as kernels address them
+    uint64_t* m_hits = nullptr;
     uint32_t* d_cursor = nullptr;
     uint8_t* d_target = nullptr;
     uint8_t* d_accum = nullptr;
@@ -93,6 +112,22 @@ struct Slot {
 };
 
 constexpr uint32_t kMaxItems = 4096;
+
+// Where a batch of `items` requests in `chunks` pieces of 64 rays has its
+// tables, from 8-byte word 0: entries, spans, offsets, then chunk items.
+struct Tables {
+    size_t spans, offsets, chunk, words;
+    Tables(size_t items, size_t chunks) {
+        static_assert(sizeof(BatchEntry) % 8 == 0 && sizeof(HostSpan) % 8 == 0, "tables are moved in 8-byte words");
+        spans = items * (sizeof(BatchEntry) / 8);
+        offsets = spans + items * (sizeof(HostSpan) / 8);
+        chunk = offsets + (items + 2) / 2;
+        words = chunk + (chunks + 1) / 2;
+    }
+    static BatchIo io(uint64_t* at, const Tables& t) {
+        return BatchIo{(BatchEntry*)at, (uint32_t*)(at + t.offsets), (uint32_t*)(at + t.chunk), nullptr};
+    }
+};
 
 }  // namespace
 
@@ -125,11 +160,10 @@ int fail(rt_server* S, int code, const std::string& m) {
 }
 
 void free_slot(Slot& s) {
-    for (void* p : {(void*)s.d_rays, (void*)s.d_hits, (void*)s.d_table, (void*)s.d_offsets, (void*)s.d_chunk,
-                    (void*)s.d_cursor, (void*)s.d_target, (void*)s.d_accum})
+    for (void* p : {(void*)s.d_rays, (void*)s.d_hits, (void*)s.d_tables, (void*)s.d_cursor, (void*)s.d_target,
+                    (void*)s.d_accum})
         if (p) (void)hipFree(p);
-    for (void* p : {(void*)s.h_rays, (void*)s.h_hits, (void*)s.h_table, (void*)s.h_offsets, (void*)s.h_chunk,
-                    (void*)s.h_target, (void*)s.h_counters})
+    for (void* p : {(void*)s.h_rays, (void*)s.h_hits, (void*)s.h_tables, (void*)s.h_target, (void*)s.h_counters})
         if (p) (void)hipHostFree(p);
     if (s.ev) (void)hipEventDestroy(s.ev);
     if (s.stream) (void)hipStreamDestroy(s.stream);
@@ -141,15 +175,17 @@ int make_slot(rt_server* S, Slot& s) {
     const uint32_t R = S->cfg.max_batch_rays, P = S->cfg.max_render_pixels;
     if (rt_create(&s.ctx, S->ctx->device) != RT_OK) return fail(S, RT_ERR_HIP, "slot context");
     if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess) return fail(S, RT_ERR_HIP, "slot stream");
-    if (hipEventCreateWithFlags(&s.ev, hipEventDisableTiming) != hipSuccess) return fail(S, RT_ERR_HIP, "slot event");
+    // (the host reads hits that kernels wrote to its memory)
+    if (hipEventCreateWithFlags(&s.ev, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess)
+        return fail(S, RT_ERR_HIP, "slot event");
     auto dm = [&](void** p, size_t b) { return hipMalloc(p, b) == hipSuccess; };
     auto hm = [&](void** p, size_t b) { return hipHostMalloc(p, b, hipHostMallocDefault) == hipSuccess; };
-    const size_t chunks = R / 64 + 2;
+    auto mm = [&](uint64_t** m, void* h) { return hipHostGetDevicePointer((void**)m, h, 0) == hipSuccess; };
+    const size_t tables = 8 * Tables(kMaxItems, R / 64 + 2).words;
     bool ok = dm((void**)&s.d_rays, (size_t)R * sizeof(rt_ray)) && dm((void**)&s.d_hits, (size_t)R * sizeof(rt_hit)) &&
               hm((void**)&s.h_rays, (size_t)R * sizeof(rt_ray)) && hm((void**)&s.h_hits, (size_t)R * sizeof(rt_hit)) &&
-              dm((void**)&s.d_table, kMaxItems * sizeof(BatchEntry)) && hm((void**)&s.h_table, kMaxItems * sizeof(BatchEntry)) &&
-              dm((void**)&s.d_offsets, (kMaxItems + 1) * 4) && hm((void**)&s.h_offsets, (kMaxItems + 1) * 4) &&
-              dm((void**)&s.d_chunk, chunks * 4) && hm((void**)&s.h_chunk, chunks * 4) && dm((void**)&s.d_cursor, 4 * kCursorBlock) &&
+              dm((void**)&s.d_tables, tables) && hm((void**)&s.h_tables, tables) &&
+              mm(&s.m_rays, s.h_rays) && mm(&s.m_hits, s.h_hits) && dm((void**)&s.d_cursor, 4 * kCursorBlock) &&
               dm((void**)&s.d_target, (size_t)P * 4) && dm((void**)&s.d_accum, (size_t)P * 4) &&
               hm((void**)&s.h_target, (size_t)P * 4) && hm((void**)&s.h_counters, 64 * 4);
     if (!ok) return fail(S, RT_ERR_NOMEM, "slot buffers");
@@ -187,20 +223,26 @@ int launch_slot(rt_server* S, Slot& sl) {
         uint32_t off = 0, need = 0;
         uint64_t long_rays = 0;     // rays on scenes of 2^17 triangles or more
         const uint32_t ni = (uint32_t)sl.reqs.size();
+        const uint32_t chunks = (uint32_t)((sl.rays + 63) / 64);
+        const Tables at(ni, chunks);
+        BatchEntry* const table = (BatchEntry*)sl.h_tables;
+        HostSpan* const spans = (HostSpan*)(sl.h_tables + at.spans);
+        uint32_t* const offsets = (uint32_t*)(sl.h_tables + at.offsets);
+        uint32_t* const chunk = (uint32_t*)(sl.h_tables + at.chunk);
         for (uint32_t i = 0; i < ni; ++i) {
             Request* r = sl.reqs[i];
             r->offset = off;
-            if (r->direct) {
+            spans[i] = r->span;
+            if (!r->direct) {
+                std::memcpy(sl.h_rays + off, r->rays, (size_t)r->n * sizeof(rt_ray));
+                spans[i].rays = sl.m_rays + (size_t)off * (sizeof(rt_ray) / 8);
+                spans[i].hits = sl.m_hits + (size_t)off * (sizeof(rt_hit) / 8);
+            } else if (!r->span.rays) {
                 if (hipMemcpyAsync(sl.d_rays + off, r->rays, (size_t)r->n * sizeof(rt_ray), hipMemcpyHostToDevice, st) !=
                     hipSuccess)
                     return RT_ERR_HIP;
-            } else {
-                std::memcpy(sl.h_rays + off, r->rays, (size_t)r->n * sizeof(rt_ray));
-                if (hipMemcpyAsync(sl.d_rays + off, sl.h_rays + off, (size_t)r->n * sizeof(rt_ray),
-                                   hipMemcpyHostToDevice, st) != hipSuccess)
-                    return RT_ERR_HIP;
             }
-            BatchEntry& e = sl.h_table[i];
+            BatchEntry& e = table[i];
             const rt_scene* sc = r->scene;
             e.nodes = sc->d_w4nodes;
             e.tris = sc->d_ptris;
@@ -214,28 +256,30 @@ int launch_slot(rt_server* S, Slot& sl) {
             e.base = off;
             e.count = r->n;
             e.win0 = 0;
-            sl.h_offsets[i] = off;
+            offsets[i] = off;
             off += r->n;
             need = std::max(need, sc->stack4);
             if (sc->info.num_triangles >= (1u << 17)) long_rays += r->n;
         }
-        sl.h_offsets[ni] = off;
-        const uint32_t chunks = (off + 63) / 64;
+        offsets[ni] = off;
         for (uint32_t i = 0, c = 0; i < ni && c < chunks; ++i)
-            while (c < chunks && (uint64_t)c * 64 < sl.h_offsets[i + 1]) sl.h_chunk[c++] = i;
-        if (hipMemcpyAsync(sl.d_table, sl.h_table, ni * sizeof(BatchEntry), hipMemcpyHostToDevice, st) != hipSuccess ||
-            hipMemcpyAsync(sl.d_offsets, sl.h_offsets, (ni + 1) * 4, hipMemcpyHostToDevice, st) != hipSuccess ||
-            hipMemcpyAsync(sl.d_chunk, sl.h_chunk, std::max(chunks, 1u) * 4, hipMemcpyHostToDevice, st) != hipSuccess)
+            while (c < chunks && (uint64_t)c * 64 < offsets[i + 1]) chunk[c++] = i;
+        if (hipMemcpyAsync(sl.d_tables, sl.h_tables, 8 * at.words, hipMemcpyHostToDevice, st) != hipSuccess)
             return RT_ERR_HIP;
-        BatchIo bio{sl.d_table, sl.d_offsets, sl.d_chunk, nullptr};
+        const BatchIo bio = Tables::io(sl.d_tables, at);
+        const HostSpan* const d_spans = (const HostSpan*)(sl.d_tables + at.spans);
+        int rc = launch_gather(sl.ctx, bio, d_spans, sl.d_rays, off, sl.d_cursor, st);
+        if (rc) return rc;
         // refill threshold as for a plain query: early refills when most rays
         // trace a large scene (long traversals), late ones otherwise
         const uint32_t refill = 2ull * long_rays >= off ? 24u : 48u;
-        int rc = launch_batch_dynamic(sl.ctx, bio, sl.d_cursor, off, need, refill, st);
+        rc = launch_batch_dynamic(sl.ctx, bio, sl.d_cursor, off, need, refill, st);
+        if (rc) return rc;
+        rc = launch_scatter(sl.ctx, bio, d_spans, sl.d_hits, off, st);
         if (rc) return rc;
         for (Request* r : sl.reqs) {
-            rt_hit* dst = r->direct ? r->hits : sl.h_hits + r->offset;
-            if (hipMemcpyAsync(dst, sl.d_hits + r->offset, (size_t)r->n * sizeof(rt_hit), hipMemcpyDeviceToHost, st) !=
+            if (!r->direct || r->span.hits) continue;
+            if (hipMemcpyAsync(r->hits, sl.d_hits + r->offset, (size_t)r->n * sizeof(rt_hit), hipMemcpyDeviceToHost, st) !=
                 hipSuccess)
                 return RT_ERR_HIP;
         }
@@ -338,6 +382,8 @@ void worker_main(rt_server* S) {
             S->st.launches++;
             lk.unlock();
             int rc = launch_slot(S, sl);
+            // what was launched may still use the requests' buffers
+            if (rc) (void)hipStreamSynchronize(sl.stream);
             lk.lock();
             if (rc) {
                 for (Request* r : sl.reqs) finish_request(S, r, rc);
@@ -589,6 +635,7 @@ extern "C" int rt_server_submit_query(rt_server* S, uint64_t scene_id, const rt_
     r->n = n;
     r->hits = hits;
     r->direct = pinned(rays) && pinned(hits);
+    if (r->direct) r->span = HostSpan{mapped(rays, (size_t)n * sizeof(rt_ray)), mapped(hits, (size_t)n * sizeof(rt_hit))};
     return submit(S, r, request_id);
 }
 
