@@ -342,22 +342,33 @@ int ensure_workspace(rt_ctx* ctx, int slot, size_t bytes);
 // lanes a wave has left over take that ray's subtrees from the first step
 // on, so few rays want many waves; but a wave pays for its steps whatever
 // its lanes do, so many rays want full ones, and a CU with one block more
-// than the others holds up the launch.  Waves per SIMD (k) were swept, us
-// per query (262,144-triangle clusters unless said):
-//   rays      16,411  65,536  131,072  262,144  400,000  1,048,576
-//   k = 2       59      92
-//   k = 3       56      87      111      158      196       366
-//   k = 4       58      89      115      147                350
-//   k = 5               95      123      154      206       335
-//   icosphere, 500k rays: camera 153 (4), 165 (5), shell 167 (4), 173 (5)
-//   1,024 triangles: 4,096 rays 20.7 (2), 21.8 (4); 65,536 44.0 (2), 48.3 (5)
+// than the others holds up the launch.  Up to 320 rays a SIMD all get their
+// lanes at the start, on up to 5 waves; a SIMD that refills its waves has 4
+// at most: with 5 the CU's waves evict each other's records from its 32 KB L1
+// between the four reads of a record (4M rays on 4M triangles: 3.1e8 reads from
+// L2 and vector units 59% busy, where 4 waves and slower code made 2.5e8 and
+// 99%).  us per query, waves per SIMD (k) swept:
+//   clusters, 262,144 triangles unless said   k = 2     3     4     5
+//     65,536 rays                                88    87
+//     131,072                                   113   107
+//     262,144 (256 rays a SIMD)                       154   140
+//     400,000                                   208   180
+//     524,288 camera                            248   186   185
+//     524,288 shell                             461   347   331
+//     1,048,576                                 427   339   303   352
+//     2,000,000 on 1M triangles                1453  1083  1104  1560
+//     the same of a camera                     1217   930   808   746
+//     4,194,304 on 4M triangles                3874  2856  2671  3679
+//   81,920-triangle icosphere, 300,000 camera   110   113   118    94
+//     500,000 shell                             164   149   156
+//   a 4k frame of 2M triangles, ms             21.0  16.6  16.0  17.8
 // and at least 4, 8 or 16 rays a wave cost 22.6, 25.0 and 29.8 us against
 // 17.3 on 256 rays: down to one a wave.
 struct LaunchPlan { uint32_t blocks, per_wave; };
 RT_HOST_DEVICE inline LaunchPlan plan_launch(uint32_t n, uint32_t grid, uint32_t waves_per_block, uint32_t simds) {
     const uint32_t load = n / simds + (n % simds != 0u);           // rays a SIMD
     uint32_t k = load <= 8u ? 2u : load <= 192u ? 3u : (load + 63u) / 64u;
-    if (load > 320u) k = (load + 64u) / 128u;
+    if (load > 320u) k = load < 448u ? 3u : 4u;
     const uint64_t want = (uint64_t)k * simds / waves_per_block;
     LaunchPlan p{want < grid ? (uint32_t)want : grid, 0u};
     // down to one ray a wave, in a number of blocks that the XCDs share evenly

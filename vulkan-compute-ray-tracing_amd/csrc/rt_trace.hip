@@ -235,19 +235,21 @@ int launch_packed_t(rt_ctx* ctx, const TraceArgs& a, hipStream_t s, bool stats) 
     // segment the ray range per XCD when there is enough of it
     const uint32_t segs = (a.n_dev || a.n >= (1u << 16)) ? kSegments : 1u;
     // 1..64 idle lanes trigger a refetch (64: only when the whole wave is
-    // idle).  The loop is bound by VALU issue, with each step's dependent
-    // record fetch close behind, so idle lanes waste issue slots and every
-    // refill stalls its wave on three dependent fetches: a large scene's long
-    // traversals want lanes refilled early, while a small scene's short ones
-    // finish so fast that each refill's fetches are better shared by more
-    // rays.  Measured from 2^17 triangles up, with the drain's
-    // work sharing taking over the lanes idle at the end: a query is best at
-    // 28 (4M-triangle query 6.06-6.08 ms against 6.10-6.11 at 24, 6.12-6.14
-    // at 32, 6.27 at 20), a render's bounces at 24 (1080p render 32.7 ms
-    // against 32.8 at 28 and 33.4 at 32).  Below 2^17 triangles 48 is best
-    // (-1..4% against 32).
+    // idle).  Idle lanes waste issue slots, and every refill stalls its wave
+    // on dependent fetches and runs the long setup of a ray: a large scene's
+    // long traversals want lanes refilled early, a small scene's short ones
+    // late.  But the more lanes are busy, the more records a CU has in flight,
+    // and past what its L1 holds every refetch is paid for in L2 requests
+    // (plan_launch), so scenes far larger than the caches want fewer.  Measured
+    // (ms at 24, 28, 32, 40, 48): 4M rays on 4M triangles 2.91 2.75 2.63 2.61
+    // 2.76; 2M box rays on 1M triangles 1.32 1.21 1.12 1.07 1.12, camera rays
+    // 0.79 0.80 0.81 0.87 0.91; 1M rays on 262,144 triangles 0.298 0.301 0.305
+    // 0.318 0.337; a 4k frame of 2M triangles 16.08 15.79 15.67 15.93 16.73.
+    // Below 2^17 triangles 48: 500,000 rays on 81,920 triangles camera 0.140
+    // 0.141 0.139 0.135 0.129, shell 0.169 0.168 0.164 0.156 0.157.
+    const uint32_t tri = sc->info.num_triangles;
     uint32_t refill = ctx->tuning.refill ? ctx->tuning.refill
-                                         : (sc->info.num_triangles >= (1u << 17) ? (a.render ? 24u : 28u) : 48u);
+                      : tri >= (1u << 19) ? 32u : tri >= (1u << 17) ? (a.render ? 32u : 28u) : 48u;
     if (refill > 64u) refill = 64u;
     TraceScene ts{sc->d_pnodes, sc->d_qnodes, sc->d_w4nodes, sc->d_ptris, sc->d_ptri_id, sc->frame,
                   LAYOUT == kLayoutW4 || LAYOUT == kLayoutW4Joined ? sc->root4 : sc->root_ref, sc->tri_off};
