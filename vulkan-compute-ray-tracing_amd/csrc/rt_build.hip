@@ -19,7 +19,7 @@
 //     positions i and j, 64 + that of the positions when the codes are
 //     equal; internal node i covers the sorted range with one end at i and
 //     splits it where the prefix shared with i ends
-//  6. boxes: leaf records, a 64-ary pyramid of box unions over the sorted
+//  6. boxes: leaf records, an 8-ary pyramid of box unions over the sorted
 //     leaves, then every internal node unions the pyramid entries that tile
 //     its leaf range (no thread waits on another, so no cross-XCD cache
 //     maintenance is needed)
@@ -191,77 +191,34 @@ __device__ inline void radix_split(const uint64_t* __restrict__ keys, int64_t N,
     g = i + s * d + (d < 0 ? -1 : 0);
 }
 
-__global__ __launch_bounds__(256) void k_radix_tree(const uint64_t* __restrict__ keys, uint32_t n,
-                                                    rt_bvh_node* __restrict__ nodes, int32_t* __restrict__ far) {
-    const int64_t N = n;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N - 1; i += (int64_t)gridDim.x * blockDim.x) {
-        int64_t j, g;
-        radix_split(keys, N, i, j, g);
-        const int64_t lo = i < j ? i : j, hi = i < j ? j : i;
-        const int32_t left = (int32_t)(lo == g ? (N - 1 + g) : g);
-        const int32_t right = (int32_t)(hi == g + 1 ? (N - 1 + g + 1) : g + 1);
-        rt_bvh_node& nd = nodes[i];
-        nd._pad0 = 0.0f;
-        nd.leftNodeIndex = left;
-        nd.rightNodeIndex = right;
-        nd.objectIndex = -1;
-        nd._pad1[0] = nd._pad1[1] = 0;
-        far[i] = (int32_t)j;                  // node i covers sorted leaves [min(i,j), max(i,j)]
-    }
-}
-
-__device__ inline void store_box(rt_bvh_node* nd, const Box& b) {
-    nd->min[0] = b.lo[0];
-    nd->min[1] = b.lo[1];
-    nd->min[2] = b.lo[2];
-    nd->max[0] = b.hi[0];
-    nd->max[1] = b.hi[1];
-    nd->max[2] = b.hi[2];
-}
-
-// Leaf records: the leaf of sorted position k is node n-1+k.
-__global__ __launch_bounds__(256) void k_leaves(const rt_triangle* __restrict__ tris, const uint32_t* __restrict__ order,
-                                                uint32_t n, rt_bvh_node* __restrict__ nodes) {
-    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-        const uint32_t tri = order[k];
-        rt_bvh_node* nd = nodes + (n - 1 + k);
-        store_box(nd, tri_box(tris, tri));
-        nd->_pad0 = 0.0f;
-        nd->leftNodeIndex = -1;
-        nd->rightNodeIndex = -1;
-        nd->objectIndex = (int32_t)tri;
-        nd->_pad1[0] = nd->_pad1[1] = 0;
-    }
-}
-
 // Box pyramid over the sorted leaves: level 0 is the leaf records, entry m
-// of level L+1 is the union of entries [64m, 64m+64) of level L.  Every
-// internal node's box is then the union of at most ~126 entries per level
-// over its leaf range -- no thread waits on another.
-constexpr int kPyramidLevels = 6;             // 64^5 > 2^30 leaves
+// of level L+1 is the union of entries [8m, 8m+8) of level L, so a leaf range
+// is tiled by at most 14 entries a level.  A wave's lanes wait for the one
+// with the most: with 8 to an entry a range of 1,000 leaves takes 56 at most,
+// with 64 it takes 126 (1M triangles, children and boxes of internal nodes: 192
+// us in two kernels with 64, 77 in one with 8; the pyramid itself 24 -> 11).
+constexpr int kFanLevels = 11;                // 8^10 = 2^30 leaves
+constexpr uint32_t kFan = 8;
+constexpr int kPyramidLevels = 6;             // rt_wide.hpp's, 64 to an entry: 64^5 = 2^30
 struct PBox {
     float4 lo, hi;
 };
 struct Pyramid {
     const rt_bvh_node* leaves;                // level 0: nodes + n - 1
-    const PBox* lvl[kPyramidLevels];          // levels 1.. (lvl[0] unused)
-    uint32_t count[kPyramidLevels];
+    PBox* lvl[kFanLevels];                    // levels 1.. (lvl[0] unused)
+    uint32_t count[kFanLevels];
     uint32_t levels;                          // levels present, level 0 included
 };
 
 __device__ inline Box pyramid_get(const Pyramid& p, uint32_t level, uint32_t k) {
-    Box b;
-    if (level == 0) {
-        const float4* q = reinterpret_cast<const float4*>(p.leaves + k);
-        const float4 lo = q[0], hi = q[1];
-        b.lo[0] = lo.x; b.lo[1] = lo.y; b.lo[2] = lo.z;
-        b.hi[0] = hi.x; b.hi[1] = hi.y; b.hi[2] = hi.z;
-    } else {
-        const PBox e = p.lvl[level][k];
-        b.lo[0] = e.lo.x; b.lo[1] = e.lo.y; b.lo[2] = e.lo.z;
-        b.hi[0] = e.hi.x; b.hi[1] = e.hi.y; b.hi[2] = e.hi.z;
-    }
-    return b;
+    const float4* q = level == 0 ? reinterpret_cast<const float4*>(p.leaves + k)
+                                 : reinterpret_cast<const float4*>(p.lvl[level] + k);
+    const float4 lo = q[0], hi = q[1];
+    return Box{{lo.x, lo.y, lo.z}, {hi.x, hi.y, hi.z}};
+}
+
+__device__ inline Box no_box() {
+    return Box{{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
 }
 
 __device__ inline void grow(Box& u, const Box& b) {
@@ -271,47 +228,94 @@ __device__ inline void grow(Box& u, const Box& b) {
     }
 }
 
-// One wave per 64-entry block of level `level` -> entry of level+1.
-__global__ __launch_bounds__(256) void k_pyramid(Pyramid p, uint32_t level, PBox* __restrict__ out) {
+// A wave's 64 entries of level `level`, from 64 * m on (b: this lane's), make
+// eight of the next level and one of the level after it.
+__device__ inline void pyramid_put(const Pyramid& p, uint32_t level, uint32_t m, Box b) {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t blocks = p.count[level + 1];
-    for (uint32_t m = (blockIdx.x * blockDim.x + threadIdx.x) / 64u; m < blocks; m += gridDim.x * blockDim.x / 64u) {
-        const uint32_t k = m * 64u + lane;
-        Box b;
-        if (k < p.count[level]) {
-            b = pyramid_get(p, level, k);
-        } else {
-            for (int a = 0; a < 3; ++a) { b.lo[a] = INFINITY; b.hi[a] = -INFINITY; }
+    for (uint32_t up = 0; up < 2 && level + 1 + up < p.levels; ++up) {
+        const int first = up == 0 ? 1 : 8, last = up == 0 ? 4 : 32;
+        for (int o = first; o <= last; o <<= 1) {
+            Box other;
+            for (int a = 0; a < 3; ++a) {
+                other.lo[a] = __shfl_xor(b.lo[a], o, 64);
+                other.hi[a] = __shfl_xor(b.hi[a], o, 64);
+            }
+            grow(b, other);
         }
-        for (int a = 0; a < 3; ++a) {
-            b.lo[a] = wave_min(b.lo[a]);
-            b.hi[a] = wave_max(b.hi[a]);
-        }
-        if (lane == 0) out[m] = PBox{make_float4(b.lo[0], b.lo[1], b.lo[2], 0.0f), make_float4(b.hi[0], b.hi[1], b.hi[2], 0.0f)};
+        const uint32_t per = up == 0 ? kFan : 64u;
+        const uint32_t at = m * (64u / per) + lane / per;
+        if (lane % per == 0 && at < p.count[level + 1 + up])
+            p.lvl[level + 1 + up][at] =
+                PBox{make_float4(b.lo[0], b.lo[1], b.lo[2], 0.0f), make_float4(b.hi[0], b.hi[1], b.hi[2], 0.0f)};
     }
 }
 
-// Internal node i's box: the union over its sorted leaf range.
-__global__ __launch_bounds__(256) void k_internal_boxes(Pyramid p, uint32_t n, const int32_t* __restrict__ far,
-                                                        rt_bvh_node* __restrict__ nodes) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i + 1 < n; i += gridDim.x * blockDim.x) {
-        const uint32_t j = (uint32_t)far[i];
-        uint32_t lo = i < j ? i : j, hi = (i < j ? j : i) + 1;    // [lo, hi) at level 0
-        Box u;
-        for (int a = 0; a < 3; ++a) { u.lo[a] = INFINITY; u.hi[a] = -INFINITY; }
+__device__ inline void store_node(rt_bvh_node* nd, const Box& b, int32_t left, int32_t right, int32_t object) {
+    float4* q = reinterpret_cast<float4*>(nd);
+    q[0] = make_float4(b.lo[0], b.lo[1], b.lo[2], 0.0f);
+    q[1] = make_float4(b.hi[0], b.hi[1], b.hi[2], __int_as_float(left));
+    q[2] = make_float4(__int_as_float(right), __int_as_float(object), 0.0f, 0.0f);
+}
+
+// Leaf records, and levels 1 and 2 while their boxes are in registers: the
+// leaf of sorted position k is node n-1+k.
+__global__ __launch_bounds__(256) void k_leaves(const rt_triangle* __restrict__ tris, const uint32_t* __restrict__ order,
+                                                uint32_t n, rt_bvh_node* __restrict__ nodes, Pyramid p) {
+    const uint32_t lane = threadIdx.x & 63u, waves = gridDim.x * blockDim.x / 64u;
+    for (uint32_t m = (blockIdx.x * blockDim.x + threadIdx.x) / 64u; m < (n + 63u) / 64u; m += waves) {
+        const uint32_t k = m * 64u + lane;
+        Box b = no_box();
+        if (k < n) {
+            const uint32_t tri = order[k];
+            b = tri_box(tris, tri);
+            store_node(nodes + (n - 1 + k), b, -1, -1, (int32_t)tri);
+        }
+        pyramid_put(p, 0, m, b);
+    }
+}
+
+// Levels level+1 and level+2 from level `level`, 64 of its entries a wave.
+__global__ __launch_bounds__(256) void k_pyramid(Pyramid p, uint32_t level) {
+    const uint32_t lane = threadIdx.x & 63u, waves = gridDim.x * blockDim.x / 64u;
+    const uint32_t count = p.count[level];
+    for (uint32_t m = (blockIdx.x * blockDim.x + threadIdx.x) / 64u; m < (count + 63u) / 64u; m += waves) {
+        const uint32_t k = m * 64u + lane;
+        pyramid_put(p, level, m, k < count ? pyramid_get(p, level, k) : no_box());
+    }
+}
+
+// Internal node i, whole: its children, and the union over its sorted leaf
+// range.  (A pass for the children and one for the boxes wrote every record's
+// lines twice and passed the ranges through memory.)
+__global__ __launch_bounds__(256) void k_internal(const uint64_t* __restrict__ keys, Pyramid p, uint32_t n,
+                                                  rt_bvh_node* __restrict__ nodes) {
+    const int64_t N = n;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N - 1; i += (int64_t)gridDim.x * blockDim.x) {
+        int64_t j, g;
+        radix_split(keys, N, i, j, g);
+        uint32_t lo = (uint32_t)(i < j ? i : j), hi = (uint32_t)(i < j ? j : i);
+        const int32_t left = (int32_t)(lo == g ? (N - 1 + g) : g);
+        const int32_t right = (int32_t)(hi == g + 1 ? (N - 1 + g + 1) : g + 1);
+        ++hi;                                                       // [lo, hi) at level 0
+        Box u = no_box();
+        // [a, b) in fours, the last one's spare reads those of its end again
+        auto take = [&](uint32_t level, uint32_t a, uint32_t b) {
+            for (uint32_t k = a; k < b; k += 4u)
+                for (uint32_t e = 0; e < 4u; ++e) grow(u, pyramid_get(p, level, min(k + e, b - 1u)));
+        };
         for (uint32_t level = 0; lo < hi; ++level) {
-            if (level + 1 == p.levels || hi - lo <= 64u) {
-                for (uint32_t k = lo; k < hi; ++k) grow(u, pyramid_get(p, level, k));
+            if (level + 1 == p.levels || hi - lo <= kFan) {
+                take(level, lo, hi);
                 break;
             }
-            const uint32_t a = min(hi, (lo + 63u) & ~63u);          // head up to a block boundary
-            const uint32_t b = max(a, hi & ~63u);                    // tail from the last boundary
-            for (uint32_t k = lo; k < a; ++k) grow(u, pyramid_get(p, level, k));
-            for (uint32_t k = b; k < hi; ++k) grow(u, pyramid_get(p, level, k));
-            lo = a / 64u;                                           // whole blocks [a, b) one level up
-            hi = b / 64u;
+            const uint32_t a = min(hi, (lo + kFan - 1u) & ~(kFan - 1u));   // head up to a block boundary
+            const uint32_t b = max(a, hi & ~(kFan - 1u));                  // tail from the last boundary
+            take(level, lo, a);
+            take(level, b, hi);
+            lo = a / kFan;                                                 // whole blocks [a, b) one level up
+            hi = b / kFan;
         }
-        store_box(nodes + i, u);
+        store_node(nodes + i, u, left, right, -1);
     }
 }
 
@@ -346,8 +350,8 @@ extern "C" int rt_bvh_build_device(rt_ctx* ctx, const rt_triangle* tris_dev, uin
     Pyramid pyr{};
     pyr.count[0] = n;
     pyr.levels = 1;
-    while (pyr.levels < (uint32_t)kPyramidLevels && pyr.count[pyr.levels - 1] > 1) {
-        pyr.count[pyr.levels] = (pyr.count[pyr.levels - 1] + 63u) / 64u;
+    while (pyr.levels < (uint32_t)kFanLevels && pyr.count[pyr.levels - 1] > 1) {
+        pyr.count[pyr.levels] = (pyr.count[pyr.levels - 1] + kFan - 1u) / kFan;
         ++pyr.levels;
     }
     size_t off = 0;
@@ -358,8 +362,7 @@ extern "C" int rt_bvh_build_device(rt_ctx* ctx, const rt_triangle* tris_dev, uin
     const size_t o_keys2 = take(sizeof(uint64_t) * n);
     const size_t o_vals = take(sizeof(uint32_t) * n);
     const size_t o_vals2 = take(sizeof(uint32_t) * n);
-    const size_t o_far = take(sizeof(int32_t) * n);
-    size_t o_lvl[kPyramidLevels] = {};
+    size_t o_lvl[kFanLevels] = {};
     for (uint32_t L = 1; L < pyr.levels; ++L) o_lvl[L] = take(sizeof(PBox) * pyr.count[L]);
     const size_t o_sort = take(sort_bytes);
     int rc = ensure_workspace(ctx, kWsBuild, off);
@@ -371,10 +374,9 @@ extern "C" int rt_bvh_build_device(rt_ctx* ctx, const rt_triangle* tris_dev, uin
     uint64_t* keys2 = (uint64_t*)(ws + o_keys2);
     uint32_t* vals = (uint32_t*)(ws + o_vals);
     uint32_t* vals2 = (uint32_t*)(ws + o_vals2);
-    int32_t* far = (int32_t*)(ws + o_far);
     void* sort_tmp = ws + o_sort;
     pyr.leaves = nodes_dev + (n - 1);
-    for (uint32_t L = 1; L < pyr.levels; ++L) pyr.lvl[L] = (const PBox*)(ws + o_lvl[L]);
+    for (uint32_t L = 1; L < pyr.levels; ++L) pyr.lvl[L] = (PBox*)(ws + o_lvl[L]);
 
     const uint32_t cap = (uint32_t)ctx->num_cus * 16u;
     const uint32_t nb = grid(n, kBoundsBlocks);
@@ -385,20 +387,14 @@ extern "C" int rt_bvh_build_device(rt_ctx* ctx, const rt_triangle* tris_dev, uin
     hipLaunchKernelGGL(k_morton, dim3(grid(n, cap)), dim3(256), 0, s, tris_dev, n, bounds, keys, vals);
     RT_HIP(ctx, hipGetLastError());
     RT_HIP(ctx, rocprim::radix_sort_pairs(sort_tmp, sort_bytes, keys, keys2, vals, vals2, n, 0u, 63u, s));
-    if (n > 1) {
-        hipLaunchKernelGGL(k_radix_tree, dim3(grid(n - 1, cap)), dim3(256), 0, s, keys2, n, nodes_dev, far);
-        RT_HIP(ctx, hipGetLastError());
-    }
-    hipLaunchKernelGGL(k_leaves, dim3(grid(n, cap)), dim3(256), 0, s, tris_dev, vals2, n, nodes_dev);
+    hipLaunchKernelGGL(k_leaves, dim3(grid(n, cap)), dim3(256), 0, s, tris_dev, vals2, n, nodes_dev, pyr);
     RT_HIP(ctx, hipGetLastError());
-    for (uint32_t L = 0; L + 1 < pyr.levels; ++L) {
-        // one wave (64 threads) per output entry
-        hipLaunchKernelGGL(k_pyramid, dim3(grid((uint64_t)pyr.count[L + 1] * 64u, cap)), dim3(256), 0, s, pyr, L,
-                           (PBox*)(ws + o_lvl[L + 1]));
+    for (uint32_t L = 2; L + 1 < pyr.levels; L += 2) {
+        hipLaunchKernelGGL(k_pyramid, dim3(grid(pyr.count[L], cap)), dim3(256), 0, s, pyr, L);
         RT_HIP(ctx, hipGetLastError());
     }
     if (n > 1) {
-        hipLaunchKernelGGL(k_internal_boxes, dim3(grid(n - 1, cap)), dim3(256), 0, s, pyr, n, far, nodes_dev);
+        hipLaunchKernelGGL(k_internal, dim3(grid(n - 1, cap)), dim3(256), 0, s, keys2, pyr, n, nodes_dev);
         RT_HIP(ctx, hipGetLastError());
     }
     return RT_OK;
