@@ -324,7 +324,7 @@ uint32_t grid(uint64_t work, uint32_t cap) {
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(g, cap));
 }
 
-size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 }  // namespace
 }  // namespace rtamd

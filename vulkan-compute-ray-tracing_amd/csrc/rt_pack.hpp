@@ -289,16 +289,18 @@ int device_pack(rt_ctx* ctx, const rt_scene_desc& d, PreparedScene& P, bool* don
     if (rc) return rc;
     hipLaunchKernelGGL(k_pack_init, dim3(1), block, 0, s, facts, counts, list, depth, cost);
     hipLaunchKernelGGL(k_pack_ranges, grid(m, 16), block, 0, s, tris, nt, d.num_materials, nodes, m, facts);
-    uint32_t h[kMaxLevels + 2] = {};
-    uint32_t level = 0, bad = 0;
+    static_assert(sizeof(PackFacts) <= sizeof(WideProgress::facts), "facts end what is read back");
+    WideProgress now{};
+    const uint32_t* h = now.counts;
+    uint32_t level = 0;
     for (;;) {
-        const uint32_t end = std::min(level + 2u * kLevelsPerSync, kMaxLevels);
+        const uint32_t end = std::min(level == 0 ? first_levels(n_max, 1) : level + 2u * kLevelsPerSync, kMaxLevels);
         for (; level < end; ++level)
             hipLaunchKernelGGL(k_pack_level, grid(n_max, 8), block, 0, s, tris, nodes, level, list, counts, depth, facts);
         RT_HIP(ctx, hipGetLastError());
-        RT_HIP(ctx, hipMemcpyAsync(h, counts, sizeof h, hipMemcpyDeviceToHost, s));
-        RT_HIP(ctx, hipMemcpyAsync(&bad, &facts->bad, 4, hipMemcpyDeviceToHost, s));
+        RT_HIP(ctx, hipMemcpyAsync(&now, counts, sizeof now, hipMemcpyDeviceToHost, s));
         RT_HIP(ctx, hipStreamSynchronize(s));
+        const bool bad = reinterpret_cast<const PackFacts*>(now.facts)->bad != 0u;
         if (bad || h[level] != 0) {
             if (bad || level == kMaxLevels) return RT_OK;
             continue;
