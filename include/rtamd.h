@@ -230,9 +230,9 @@ typedef struct rt_tuning {
     uint32_t node_layout;   /* RT_LAYOUT_*: binary 64-byte fp32 or 32-byte 16-bit
                                nodes, or 4-wide 64-byte 16-bit nodes            */
     uint32_t refill;        /* idle lanes (1..64) that make a wave fetch rays;
-                               0 = by scene: from 2^17 triangles up (long
-                               traversals) 28 for queries and 24 for render
-                               bounces, 48 below (short ones)                    */
+                               0 = by scene: 48 below 2^17 triangles (short
+                               traversals), above (long ones) 36 for render
+                               bounces, 28 for queries, 40 for them from 2^19 up */
     uint32_t blocks_per_cu; /* persistent blocks per CU (0 = occupancy limit)     */
     uint32_t stack_lds;     /* 4-wide layout: 0 = the whole traversal stack in LDS
                                where the launch's blocks fit a CU like that, else

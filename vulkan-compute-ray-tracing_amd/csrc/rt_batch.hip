@@ -668,7 +668,7 @@ extern "C" int rt_batch_autotune(rt_ctx* ctx, rt_batch* b, uint32_t trials, cons
     float cur_ms = 0.0f;
     int rc = time_cfg(cur, cur_ms);
     // coordinate descent over: work-group size, node-fetch layout (4-wide or
-    // binary 16-bit records), LDS stack ring, regrouping (off, origin cell,
+    // binary 16-bit records), stack entries in LDS, regrouping (off, origin cell,
     // direction octant + origin cell), regroup interval, refill threshold
     // and blocks per CU
     const std::vector<uint32_t> blocks = {256, 128}, layouts = {RT_LAYOUT_W4, RT_LAYOUT_Q16},

@@ -241,15 +241,16 @@ int launch_packed_t(rt_ctx* ctx, const TraceArgs& a, hipStream_t s, bool stats) 
     // late.  But the more lanes are busy, the more records a CU has in flight,
     // and past what its L1 holds every refetch is paid for in L2 requests
     // (plan_launch), so scenes far larger than the caches want fewer.  Measured
-    // (ms at 24, 28, 32, 40, 48): 4M rays on 4M triangles 2.91 2.75 2.63 2.61
-    // 2.76; 2M box rays on 1M triangles 1.32 1.21 1.12 1.07 1.12, camera rays
-    // 0.79 0.80 0.81 0.87 0.91; 1M rays on 262,144 triangles 0.298 0.301 0.305
-    // 0.318 0.337; a 4k frame of 2M triangles 16.08 15.79 15.67 15.93 16.73.
-    // Below 2^17 triangles 48: 500,000 rays on 81,920 triangles camera 0.140
-    // 0.141 0.139 0.135 0.129, shell 0.169 0.168 0.164 0.156 0.157.
+    // (ms at 28, 32, 36, 40, 44): 4M rays on 4M triangles 2.93 2.75 2.65 2.61
+    // 2.63; 2M box rays on 1M triangles 1.33 1.21 1.12 1.09 1.06, camera rays
+    // 0.76 0.78 0.81 0.83 0.85; 1M rays on 262,144 triangles 0.294 0.294 0.304
+    // 0.307 0.324; a 1080p frame of 4M triangles, 4 samples, 15.90 15.64 15.56
+    // 15.59 15.83.  Below 2^17 triangles 48: 500,000 rays on 81,920 triangles
+    // at 24, 28, 32, 40, 48 camera 0.140 0.141 0.139 0.135 0.129, shell 0.169
+    // 0.168 0.164 0.156 0.157.
     const uint32_t tri = sc->info.num_triangles;
     uint32_t refill = ctx->tuning.refill ? ctx->tuning.refill
-                      : tri >= (1u << 19) ? 32u : tri >= (1u << 17) ? (a.render ? 32u : 28u) : 48u;
+                      : tri < (1u << 17) ? 48u : a.render ? 36u : tri < (1u << 19) ? 28u : 40u;
     if (refill > 64u) refill = 64u;
     TraceScene ts{sc->d_pnodes, sc->d_qnodes, sc->d_w4nodes, sc->d_ptris, sc->d_ptri_id, sc->frame,
                   LAYOUT == kLayoutW4 || LAYOUT == kLayoutW4Joined ? sc->root4 : sc->root_ref, sc->tri_off};

@@ -326,10 +326,11 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
     // step.  A wave's rays end one or two at a time, so every other step would
     // go through that code for them, id fetch included.  With the steps in a
     // loop of their own below, whose few values stay in their registers, a 4M-ray
-    // query issues 1.21e9 vector instructions instead of 1.45e9.  us before and
+    // query issued 1.21e9 vector instructions instead of 1.45e9.  us before and
     // after, with the launch shapes and refill thresholds that suit it: that
     // query 2,716 -> 2,634; 1M rays on 262,144 triangles 325 -> 301; 500,000
-    // on an 81,920-triangle icosphere 168 -> 156; a 4k frame 16,260 -> 15,670.
+    // on an 81,920-triangle icosphere 168 -> 156; a 1080p frame
+    // of 4 samples 16,260 -> 15,670.
     constexpr int32_t kIdle = 0;        // no ray
     constexpr int32_t kBusy = 1;        // takes steps
     constexpr int32_t kStopped = 2;     // its traversal has ended
@@ -377,7 +378,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
     // 300,000 122 -> 97, 524,288 149 -> 133; on 262,144-triangle clusters
     // 65,536 100 -> 74, 524,288 212 -> 198.  Rays without order pay for the
     // scattered reads: 0 to 2% (65,536 on 1,024 triangles 44.0 -> 46.7).  Not
-    // where waves take whole chunks (a 4k frame is the same either way: there
+    // where waves take whole chunks (a 1080p frame of 4 samples is the same either way: there
     // are enough rays to even the waves out), and not in a render's bounces
     // that use the cursors (four 960x540 frames 1,200 -> 1,240).
     const uint32_t deal = !BATCHED && io.deal && !fits && !chunked && !io.order ? n / 64u * kDealRun : 0u;
@@ -496,19 +497,23 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                 float k0 = __builtin_inff(), k1 = __builtin_inff(), k2 = __builtin_inff(), k3 = __builtin_inff();
                 float tn;
                 int nh = 0;
-                // child k's words: entry and exit planes by the ray's selectors
-                auto box = [&](uint32_t wx, uint32_t wy, uint32_t wz, float& key) {
-                    if (slab_ordered(biased_plane(wx, sn_x), biased_plane(wy, sn_y), biased_plane(wz, sn_z),
-                                     biased_plane(wx, sf_x), biased_plane(wy, sf_y), biased_plane(wz, sf_z), cq,
-                                     inv, tmin_rel, best_rel, tn)) {
+                // child k's words: entry and exit planes by the ray's
+                // selectors.  An unused slot is tested too and masked: some
+                // lane has a child there in nearly every step, so a branch
+                // around the test saves nothing (16,411 rays 52.1 -> 50.8 us,
+                // 500,000 157 -> 153, 1M on 60,000 triangles 613 -> 592).
+                auto box = [&](uint32_t wx, uint32_t wy, uint32_t wz, bool used, float& key) {
+                    if (used & slab_ordered(biased_plane(wx, sn_x), biased_plane(wy, sn_y), biased_plane(wz, sn_z),
+                                            biased_plane(wx, sf_x), biased_plane(wy, sf_y), biased_plane(wz, sf_z),
+                                            cq, inv, tmin_rel, best_rel, tn)) {
                         key = tn;
                         nh++;
                     }
                 };
-                if (d.x != kNoChild) box(a.x, a.y, a.z, k0);
-                if (d.y != kNoChild) box(a.w, b.x, b.y, k1);
-                if (d.z != kNoChild) box(b.z, b.w, c.x, k2);
-                if (d.w != kNoChild) box(c.y, c.z, c.w, k3);
+                box(a.x, a.y, a.z, d.x != kNoChild, k0);
+                box(a.w, b.x, b.y, d.y != kNoChild, k1);
+                box(b.z, b.w, c.x, d.z != kNoChild, k2);
+                box(c.y, c.z, c.w, d.w != kNoChild, k3);
                 if (nh > 0) {
                     int32_t v0 = d.x, v1 = d.y, v2 = d.z, v3 = d.w;
                     // sort the four (entry distance, child) pairs; misses carry +inf
@@ -517,7 +522,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                     cswap(k0, v0, k2, v2);
                     // (leaving out the last two exchanges, so that all but the
                     // nearest stay unsorted, costs more steps than it saves:
-                    // a 4k frame 16.1 -> 16.9 ms)
+                    // a 1080p frame of 4 samples 16.1 -> 16.9 ms)
                     cswap(k1, v1, k3, v3);
                     cswap(k1, v1, k2, v2);
                     // farthest pushed first so the nearest deferred child pops first
