@@ -136,9 +136,10 @@ def add_counter_rows(agg: dict, rows, k: int):
         dd["c"][row.get("Counter_Name", "")] = float(row.get("Counter_Value", 0) or 0)
         if row.get("Start_Timestamp") and row.get("End_Timestamp"):
             dd["ns"] = float(row["End_Timestamp"]) - float(row["Start_Timestamp"])
-    # the calibration copy is the class's largest dispatch (other copies are small transfers)
-    big_copy = max((key for (cls, key) in per if cls == "copy"), key=lambda kk: per[("copy", kk)]["grid"],
-                   default=None)
+    # the calibration copy is the class's largest dispatch: of those with the
+    # largest grid (an upload's copies fill it too) the one that counted most
+    big_copy = max((key for (cls, key) in per if cls == "copy"),
+                   key=lambda kk: (per[("copy", kk)]["grid"], sum(per[("copy", kk)]["c"].values())), default=None)
     for (cls, key), dd in per.items():
         if cls == "copy" and key != big_copy:
             continue
