@@ -74,6 +74,7 @@ static_assert(sizeof(PNodeQ) == 32, "quantized node record");
 struct alignas(16) PNode4 { uint32_t w[12]; int32_t ref[4]; };
 static_assert(sizeof(PNode4) == 64, "4-wide node record");
 constexpr int32_t kNoChild = INT32_MIN + 1;
+constexpr int32_t kPassed = INT32_MIN + 2;      // never stored: a child that a second trace does not enter
 
 // Fixed-point frame of the quantized nodes, with 1/scale for the rays in
 // binary32 and binary64 (a ray's setup takes products, not divisions).

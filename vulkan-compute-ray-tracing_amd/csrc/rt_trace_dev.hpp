@@ -297,12 +297,20 @@ __device__ __forceinline__ float shfl_f(float x, uint32_t src) {
 // tree names the one reported: the first in the order in which a traversal
 // of its records alone visits them.  This loop walks another tree
 // (rt_scene::root4) in shared pieces, so it only notes that its closest t
-// was met twice (`tie`); every box that holds a hit at the closest t is
+// was met twice (kTied); every box that holds a hit at the closest t is
 // visited, so no tie is missed.  A ray that ends with a tie is traced again
-// by one lane (`exact`) through the caller's records, whose root is record
-// 0, with its closest t as an inclusive bound: only boxes up to that t are
-// visited, in the order of a full traversal (a child's place among its
-// siblings depends on entry distances alone), and the first hit met is kept.
+// by one lane through the caller's records, whose root is record 0, and the
+// first hit at its closest t that it meets is kept.  It enters only the boxes
+// that hold the hit's point, within hit_slack, in the order of a full traversal
+// (a child's place among its siblings depends on entry distances alone; those
+// not entered are sorted with the others).  A hit whose t the triangle test
+// rounded by more than the slack, on a surface seen nearly edge on, may lie
+// outside its own boxes there: a trace that meets nothing is made over all
+// boxes of the ray, and if that too meets nothing the first trace's hit stands.
+// us for 1M rays, each triangle given once, given twice so that every hit is a
+// tie, and that with a second trace over all that lies before the hit: a
+// 20,480-triangle icosphere (28% hits) 154, 244, 386; 131,072 triangles in
+// clusters (6%) 221, 266, 480.
 template <int BLOCK, int STACK, int LAYOUT, bool STATS, bool BATCHED, bool DEEP>
 __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const TraceIo& io, const BatchIo& bio,
                                                  int32_t* __restrict__ stk, int32_t* __restrict__ spill) {
@@ -335,6 +343,12 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
     constexpr int32_t kBusy = 1;        // takes steps
     constexpr int32_t kStopped = 2;     // its traversal has ended
     constexpr int32_t kWaiting = 3;     // drained waves: so has it, but its helpers are busy
+    // Which trace of its ray a lane is at (see Ties).
+    constexpr int32_t kFirst = 0;       // first trace
+    constexpr int32_t kTied = 1;        // so far its closest t was met by two triangles
+    constexpr int32_t kNearHit = 2;     // second trace, boxes that hold the closest hit's point
+    constexpr int32_t kWholeRay = 3;    // second trace, every box that the ray meets
+    constexpr int32_t kMet = 4;         // it has met the hit
     int32_t state = kIdle;
     bool drained = false;           // wave-uniform: every segment is used up
     // Segments: the ray range (all items' rays, for batched launches) is cut into io.segs
@@ -401,7 +415,8 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
     };
     f3 cq{0.0f, 0.0f, 0.0f};        // plane_bias: 4-wide box planes are biased_plane * inv + cq
     // node tests run on t - t_shift (frame_far); tmin_rel and best_rel are
-    // tmin and the closest hit's t on that scale (equal to them when t_shift = 0)
+    // tmin and the closest hit's t on that scale (equal to them when t_shift = 0,
+    // else best_rel is rel_bound's)
     float t_shift = 0.0f, tmin_rel = 0.0f, best_rel = 0.0f;
     float best_t = 0.0f, bu = 0.0f, bv = 0.0f;
     int32_t best = -1;
@@ -409,8 +424,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
     uint64_t sum_nv = 0, sum_nt = 0;   // STATS: this lane's totals over its rays
     int sp = 0;
     int32_t cur = 0;
-    bool tie = false;               // best_t was met by two triangles
-    bool exact = false;             // second trace of a tied ray, through the caller's records
+    int32_t stage = kFirst;
     // work sharing (STEAL): the stack holds entries [bot, sp)
     int bot = 0;
     int32_t owner = -1;             // a helper's owner lane; -1 for the owner
@@ -442,10 +456,19 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
         return v;
     };
 
+    // The closest t as a bound of the boxes.  A far ray's t carries the rounding
+    // of |t|, its boxes only that of t - t_shift: the bound is let out by as
+    // much, or the box of a second triangle at the same t may lie past it.
+    auto rel_bound = [&](float t) { return __builtin_fmaf(fabsf(t_shift), 0x1p-17f, t - t_shift); };
+    // How far from its computed t a second trace looks for the hit it knows of.
+    auto hit_slack = [&]() { return fabsf(best_t) * 0x1p-12f; };
+
     // ---- one traversal step per busy lane
     auto step = [&]() {
         if (state != kBusy) return;
         const bool deep = DEEP && __ballot(sp > STACK - 3) != 0;
+        // likewise whether any lane is at its second trace
+        const bool seconds = kW4 && __ballot(stage >= kNearHit) != 0;
         bool next = false;          // cur holds the next record to read
         if constexpr (kW4) {
             // One memory round trip per step whatever the lanes' mix of
@@ -492,8 +515,27 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
             asm volatile("" : "+v"(dw));
             asm volatile("" : "+v"(a), "+v"(b), "+v"(c));
             if (node) {
-                const int4 d = make_int4((int)dw.x, (int)dw.y, (int)dw.z, (int)dw.w);
+                int4 d = make_int4((int)dw.x, (int)dw.y, (int)dw.z, (int)dw.w);
                 if (STATS) nv++;
+                if (seconds && stage == kNearHit) {
+                    // boxes left before the hit keep their places in the
+                    // order, but are not entered
+                    const float from = best_rel - 2.0f * hit_slack();
+                    // (other names for the selectors, or the compiler keeps
+                    // these planes for the box tests in 11 more registers)
+                    uint32_t ex = sf_x, ey = sf_y, ez = sf_z;
+                    asm("" : "+v"(ex), "+v"(ey), "+v"(ez));
+                    auto left = [&](uint32_t wx, uint32_t wy, uint32_t wz, int32_t& child) {
+                        const float fx = __builtin_fmaf(biased_plane(wx, ex), inv.x, cq.x);
+                        const float fy = __builtin_fmaf(biased_plane(wy, ey), inv.y, cq.y);
+                        const float fz = __builtin_fmaf(biased_plane(wz, ez), inv.z, cq.z);
+                        if (fminf(fminf(fx, fy), fz) < from && child != kNoChild) child = kPassed;
+                    };
+                    left(a.x, a.y, a.z, d.x);
+                    left(a.w, b.x, b.y, d.y);
+                    left(b.z, b.w, c.x, d.z);
+                    left(c.y, c.z, c.w, d.w);
+                }
                 float k0 = __builtin_inff(), k1 = __builtin_inff(), k2 = __builtin_inff(), k3 = __builtin_inff();
                 float tn;
                 int nh = 0;
@@ -525,6 +567,13 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                     // a 1080p frame of 4 samples 16.1 -> 16.9 ms)
                     cswap(k1, v1, k3, v3);
                     cswap(k1, v1, k2, v2);
+                    if (seconds && stage == kNearHit) {
+                        // (boxes missed sort last, so the nh met come first)
+                        if (nh > 3 && v3 == kPassed) nh = 3;
+                        if (nh > 2 && v2 == kPassed) { v2 = v3; --nh; }
+                        if (nh > 1 && v1 == kPassed) { v1 = v2; v2 = v3; --nh; }
+                        if (v0 == kPassed) { v0 = v1; v1 = v2; v2 = v3; --nh; }
+                    }
                     // farthest pushed first so the nearest deferred child pops first
                     if (deep) {
                         if (nh > 3) push(v3, true);
@@ -536,7 +585,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                         if (nh > 1) push(v1, false);
                     }
                     cur = v0;
-                    next = true;
+                    next = nh > 0;
                 }
             } else {
                 const int32_t slot = ~cur;
@@ -550,12 +599,13 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                 float t, u, v;
                 if (tri_meets(tr, r.o, r.d, r.tmin, t, u, v)) {
                     const bool equal = t == best_t;
-                    if (t < best_t || (equal && exact && best < 0)) {
+                    if (t < best_t || (equal && (stage == kNearHit || stage == kWholeRay))) {
                         best_t = t; bu = u; bv = v; best = slot;
-                        best_rel = t - t_shift;
-                        tie = false;
-                    } else if (equal && best >= 0) {
-                        tie = true;
+                        best_rel = rel_bound(t);
+                        stage = stage < kNearHit ? kFirst : kMet;
+                        if (stage == kMet) sp = bot;      // nothing more to look for
+                    } else if (equal && best >= 0 && stage == kFirst) {
+                        stage = kTied;
                     }
                 }
             }
@@ -613,9 +663,9 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
     // ---- a lane whose traversal has ended: a tied ray's second trace begins
     // (false), or its hit is due (spheres follow in their own pass)
     auto has_hit = [&]() -> bool {
-        if (kW4 && tie && !exact) {
-            exact = true;                   // best_t and best_rel stay as bounds
-            best = -1;
+        if (kW4 && stage != kFirst && stage < kWholeRay) {
+            ++stage;
+            best_rel = stage == kNearHit ? best_rel + hit_slack() : __builtin_inff();
             cur = 0;
             sp = 0;
             bot = 0;
@@ -747,7 +797,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                     best_rel = r.tmax - t_shift;
                     best_t = r.tmax; bu = 0.0f; bv = 0.0f; best = -1;
                     nv = 0; nt = 0; sp = 0;
-                    tie = false; exact = false;
+                    stage = kFirst;
                     bot = 0; owner = -1; pending = 0;
                     cur = root;
                     // an empty tree, or a ray that misses the frame's box
@@ -774,7 +824,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                 const float owner_rel = shfl_f(best_rel, owner < 0 ? lane : (uint32_t)owner);
                 if (state == kBusy && owner >= 0) best_rel = fminf(best_rel, owner_rel);
                 const uint64_t idle_m = __ballot(state == kIdle);
-                const uint64_t donor_m = __ballot(state == kBusy && !exact && sp - bot >= 1 && (!DEEP || bot < STACK));
+                const uint64_t donor_m = __ballot(state == kBusy && stage < kNearHit && sp - bot >= 1 && (!DEEP || bot < STACK));
                 if ((uint32_t)__popcll(idle_m) >= io.steal && donor_m != 0) {
                     const uint32_t k = min((uint32_t)__popcll(idle_m), (uint32_t)__popcll(donor_m));
                     const uint32_t rank_idle = (uint32_t)__popcll(idle_m & lanes_below);
@@ -792,9 +842,9 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                     const float bestr = shfl_f(best_rel, src), bestt = shfl_f(best_t, src);
                     const int v_bot = __shfl(bot, (int)src);
                     const float v_bu = shfl_f(bu, src), v_bv = shfl_f(bv, src);
-                    // its hit, and whether its t was met twice
+                    // its hit, and whether that t was met twice
                     const int32_t v_best = __shfl(best, (int)src);
-                    const int v_tie = __shfl((int)tie, (int)src);
+                    const int32_t v_stage = __shfl(stage, (int)src);
                     const int32_t v_owner = __shfl(owner < 0 ? (int32_t)lane : owner, (int)src);
                     // batched lanes each carry their item's scene
                     auto shfl_ptr = [&](const void* q) -> uint64_t {
@@ -828,8 +878,7 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                         best_rel = bestr;
                         best_t = bestt;
                         bu = v_bu; bv = v_bv; best = v_best;
-                        tie = v_tie != 0;
-                        exact = false;
+                        stage = v_stage;
                         sp = 0; bot = 0;
                         owner = v_owner;
                         pending = 0;
@@ -864,16 +913,16 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                     const float ht = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(best_t), j));
                     const float hu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bu), j));
                     const float hv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bv), j));
-                    const bool htie = __builtin_amdgcn_readlane((int)tie, j) != 0;
+                    const int32_t h_stage = __builtin_amdgcn_readlane(stage, j);
                     if ((int32_t)lane == o) {
                         pending--;
                         // (a helper may bring back the hit it started from)
                         if (hb >= 0 && ht < best_t) {
                             best = hb; best_t = ht; bu = hu; bv = hv;
-                            best_rel = ht - t_shift;
-                            tie = htie;
+                            best_rel = rel_bound(ht);
+                            stage = h_stage;
                         } else if (hb >= 0 && ht == best_t) {
-                            tie = tie || htie || hb != best;
+                            stage = hb != best ? kTied : max(stage, h_stage);
                         }
                     }
                 }
