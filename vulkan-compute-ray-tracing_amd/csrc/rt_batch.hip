@@ -253,6 +253,7 @@ struct rt_batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     uint64_t tuning_gen = 0;           // the context's tuning the launch was set up under
+    bool ready = false;                // set up for cfg: a set-up that failed must not be launched
 };
 
 namespace {
@@ -273,6 +274,7 @@ int launch_batch_kernel(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
             RT_HIP(ctx, hipDeviceSynchronize());
             if (b->d_spill) RT_HIP(ctx, hipFree(b->d_spill));
             b->d_spill = nullptr;
+            b->spill_bytes = 0;
             RT_HIP(ctx, hipMalloc((void**)&b->d_spill, bytes));
             b->spill_bytes = bytes;
         }
@@ -303,14 +305,17 @@ int launch_batch_binary(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
 template <int BLOCK>
 int launch_batch_block(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
     if (binary_layout(b->cfg)) return launch_batch_binary<BLOCK>(ctx, b, s);
-    // the first entries of each lane's stack in LDS, the rest in b->d_spill
     const uint32_t need = b->stack_need;
     if (need > kMaxWideStack) return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: a 4-wide tree deeper than 31 levels");
-    if (need <= kStackLds) return launch_batch_kernel<BLOCK, kStackLds, false, kLayoutW4>(ctx, b, s);
-    if (b->cfg.stack_lds == 8) return launch_batch_kernel<BLOCK, 8, true, kLayoutW4>(ctx, b, s);
-    if (b->cfg.stack_lds == 16) return launch_batch_kernel<BLOCK, 16, true, kLayoutW4>(ctx, b, s);
-    if (b->cfg.stack_lds == 32) return launch_batch_kernel<BLOCK, 32, true, kLayoutW4>(ctx, b, s);
-    return launch_batch_kernel<BLOCK, kStackLds, true, kLayoutW4>(ctx, b, s);
+    const StackPlan p = plan_stack(need, b->cfg.stack_lds, true);
+    if (!p.deep) {
+        if (p.lds == 24) return launch_batch_kernel<BLOCK, 24, false, kLayoutW4>(ctx, b, s);
+        return launch_batch_kernel<BLOCK, 36, false, kLayoutW4>(ctx, b, s);     // 32 asked for, and enough
+    }
+    if (p.lds == 8) return launch_batch_kernel<BLOCK, 8, true, kLayoutW4>(ctx, b, s);
+    if (p.lds == 16) return launch_batch_kernel<BLOCK, 16, true, kLayoutW4>(ctx, b, s);
+    if (p.lds == 32) return launch_batch_kernel<BLOCK, 32, true, kLayoutW4>(ctx, b, s);
+    return launch_batch_kernel<BLOCK, 24, true, kLayoutW4>(ctx, b, s);
 }
 
 // The whole launch sequence on `s` (also what the graph captures).
@@ -378,6 +383,7 @@ int prepare_table(rt_ctx* ctx, rt_batch* b) {
 // the sequence into a graph when the configuration asks for one.
 int capture(rt_ctx* ctx, rt_batch* b) {
     drop_graph(b);
+    b->ready = false;
     int trc = prepare_table(ctx, b);
     if (trc) return trc;
     b->tuning_gen = ctx->tuning_gen;
@@ -385,7 +391,10 @@ int capture(rt_ctx* ctx, rt_batch* b) {
     int rc = launch_sequence(ctx, b, nullptr);
     b->dry = false;
     if (rc) return rc;
-    if (!b->cfg.use_graph || b->total == 0) return RT_OK;
+    if (!b->cfg.use_graph || b->total == 0) {
+        b->ready = true;
+        return RT_OK;
+    }
     RT_HIP(ctx, hipStreamBeginCapture(b->cap_stream, hipStreamCaptureModeThreadLocal));
     rc = launch_sequence(ctx, b, b->cap_stream);
     hipGraph_t g = nullptr;
@@ -397,6 +406,7 @@ int capture(rt_ctx* ctx, rt_batch* b) {
     if (e != hipSuccess) return hip_error(ctx, e, "hipStreamEndCapture");
     b->graph = g;
     RT_HIP(ctx, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
+    b->ready = true;
     return RT_OK;
 }
 
@@ -580,7 +590,7 @@ extern "C" int rt_batch_launch(rt_ctx* ctx, rt_batch* b, void* stream) {
     hipStream_t s = (hipStream_t)stream;
     // the context's tuning (the drain's steal threshold) changed since the
     // launch was set up: set it up again, so a replay never runs stale values
-    if (b->tuning_gen != ctx->tuning_gen) {
+    if (!b->ready || b->tuning_gen != ctx->tuning_gen) {
         const int rc = capture(ctx, b);
         if (rc) return rc;
     }

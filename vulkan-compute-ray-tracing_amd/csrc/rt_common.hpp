@@ -382,6 +382,18 @@ RT_HOST_DEVICE inline LaunchPlan plan_launch(uint32_t n, uint32_t grid, uint32_t
     return p;
 }
 
+// Where a 4-wide launch keeps its lanes' stacks of up to `need` entries: the
+// first `lds` in LDS, the rest (deep) in a spill area.
+struct StackPlan { uint32_t lds; bool deep; };
+// `asked`: rt_tuning's or rt_batch_config's stack_lds; `crowded`: without one,
+// the launch's blocks fit a CU only with the first kStackLds entries in LDS.
+inline StackPlan plan_stack(uint32_t need, uint32_t asked, bool crowded) {
+    if (asked && asked < need) return {asked, true};
+    if (!asked && crowded && need > kStackLds) return {kStackLds, true};
+    return {need <= kStackLds ? kStackLds : need <= 36u ? 36u : need <= 48u ? 48u : need <= 64u ? 64u : kMaxWideStack,
+            false};
+}
+
 // Launchers (rt_trace.hip).
 struct TraceArgs {
     const rt_scene* scene;
