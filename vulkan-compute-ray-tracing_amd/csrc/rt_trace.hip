@@ -389,18 +389,17 @@ int launch_trace_packed(rt_ctx* ctx, const TraceArgs& a, hipStream_t s) {
         const uint32_t expect = a.expect ? a.expect : a.n;
         const uint32_t want = (plan_launch(expect, cus * 5u, kBlock / 64, device_simds(ctx)).blocks + cus - 1u) / cus;
         const uint32_t lds = ctx->tuning.stack_lds;
-        int rc = kNoSpill;
-        if (lds && lds < need) {
-            if (a.no_alloc)
-                return set_error(ctx, RT_ERR_UNSUPPORTED, "a partial LDS stack spills to a workspace: set stack_lds to 0");
-            if (lds == 8) rc = launch_w4<8, true>(ctx, a, s, stats);
-            else if (lds == 16) rc = launch_w4<16, true>(ctx, a, s, stats);
-            else rc = launch_w4<32, true>(ctx, a, s, stats);
-        } else if (need > kStackLds && want > whole_stack_blocks(need) && !a.no_alloc) {
-            rc = launch_w4<kStackLds, true>(ctx, a, s, stats);
+        if (a.no_alloc && lds && lds < need)
+            return set_error(ctx, RT_ERR_UNSUPPORTED, "a partial LDS stack spills to a workspace: set stack_lds to 0");
+        const StackPlan p = plan_stack(need, lds, want > whole_stack_blocks(need) && !a.no_alloc);
+        if (p.deep) {
+            const int rc = p.lds == 8    ? launch_w4<8, true>(ctx, a, s, stats)
+                           : p.lds == 16 ? launch_w4<16, true>(ctx, a, s, stats)
+                           : p.lds == 32 ? launch_w4<32, true>(ctx, a, s, stats)
+                                         : launch_w4<kStackLds, true>(ctx, a, s, stats);
+            // (no spill area during a capture that comes before the area exists)
+            if (rc != kNoSpill) return rc;
         }
-        // (no spill area during a capture that comes before the area exists)
-        if (rc != kNoSpill) return rc;
         if (need <= kStackLds) return launch_w4<kStackLds, false>(ctx, a, s, stats);
         if (need <= 36) return launch_w4<36, false>(ctx, a, s, stats);
         if (need <= 48) return launch_w4<48, false>(ctx, a, s, stats);
