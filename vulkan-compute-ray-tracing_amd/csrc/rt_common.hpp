@@ -247,6 +247,7 @@ struct rt_scene {
     int32_t root4 = rtamd::kEmptyRoot;
     bool wide = false;
     uint32_t stack4 = 0;              // stack entries either tree needs, plus one
+    uint32_t given_stack4 = 0;        // the caller's records alone
     rtamd::PTri* d_ptris = nullptr;
     // d_w4nodes and d_ptris share one allocation when both fit in 4 GiB:
     // d_ptris = d_w4nodes + tri_off bytes, so a kernel addresses either

@@ -731,6 +731,7 @@ int scene_commit(rt_ctx* ctx, PreparedScene& P, rt_scene** out) {
     s->frame = packed.frame;
     s->root4 = !fast ? kEmptyRoot : s->wide ? (int32_t)P.given_records : packed.root4;
     s->stack4 = fast ? std::max(packed.stack4, P.wide_need) : 0;
+    s->given_stack4 = fast ? packed.stack4 : 0;
     P.wide.reset();
     s->packed_height = fast ? packed.height : 0;
     s->ref_height = P.chk.height;

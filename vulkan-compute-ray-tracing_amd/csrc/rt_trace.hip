@@ -389,9 +389,10 @@ int launch_trace_packed(rt_ctx* ctx, const TraceArgs& a, hipStream_t s) {
         const uint32_t expect = a.expect ? a.expect : a.n;
         const uint32_t want = (plan_launch(expect, cus * 5u, kBlock / 64, device_simds(ctx)).blocks + cus - 1u) / cus;
         const uint32_t lds = ctx->tuning.stack_lds;
-        if (a.no_alloc && lds && lds < need)
+        // (the scene's own tree decides, not the one built at upload)
+        if (a.no_alloc && lds && (lds < kStackLds || sc->given_stack4 > kStackLds))
             return set_error(ctx, RT_ERR_UNSUPPORTED, "a partial LDS stack spills to a workspace: set stack_lds to 0");
-        const StackPlan p = plan_stack(need, lds, want > whole_stack_blocks(need) && !a.no_alloc);
+        const StackPlan p = plan_stack(need, a.no_alloc ? 0u : lds, want > whole_stack_blocks(need) && !a.no_alloc);
         if (p.deep) {
             const int rc = p.lds == 8    ? launch_w4<8, true>(ctx, a, s, stats)
                            : p.lds == 16 ? launch_w4<16, true>(ctx, a, s, stats)
