@@ -249,6 +249,7 @@ struct rt_batch {
     uint32_t packed_height = 0;        // deepest binary tree among the items (binary records)
     uint32_t grid_blocks = 0;          // persistent blocks for cfg (set by a dry pass)
     bool dry = false;                  // size buffers only, launch nothing
+    bool whole_stacks = false;         // no memory for cfg's spill area: whole stacks in LDS
     hipStream_t cap_stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -275,7 +276,11 @@ int launch_batch_kernel(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
             if (b->d_spill) RT_HIP(ctx, hipFree(b->d_spill));
             b->d_spill = nullptr;
             b->spill_bytes = 0;
-            RT_HIP(ctx, hipMalloc((void**)&b->d_spill, bytes));
+            if (hipMalloc((void**)&b->d_spill, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                b->d_spill = nullptr;
+                return kNoSpill;
+            }
             b->spill_bytes = bytes;
         }
         return RT_OK;
@@ -302,20 +307,28 @@ int launch_batch_binary(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
     return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: a binary tree deeper than 64 levels");
 }
 
+static_assert(kStackLds == 24 && kMaxWideStack == 96, "the variants below");
+
 template <int BLOCK>
 int launch_batch_block(rt_ctx* ctx, rt_batch* b, hipStream_t s) {
     if (binary_layout(b->cfg)) return launch_batch_binary<BLOCK>(ctx, b, s);
     const uint32_t need = b->stack_need;
     if (need > kMaxWideStack) return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: a 4-wide tree deeper than 31 levels");
+    if (b->dry) b->whole_stacks = false;
     const StackPlan p = plan_stack(need, b->cfg.stack_lds, true);
-    if (!p.deep) {
-        if (p.lds == 24) return launch_batch_kernel<BLOCK, 24, false, kLayoutW4>(ctx, b, s);
-        return launch_batch_kernel<BLOCK, 36, false, kLayoutW4>(ctx, b, s);     // 32 asked for, and enough
+    if (p.deep && !b->whole_stacks) {
+        const int rc = p.lds == 8    ? launch_batch_kernel<BLOCK, 8, true, kLayoutW4>(ctx, b, s)
+                       : p.lds == 16 ? launch_batch_kernel<BLOCK, 16, true, kLayoutW4>(ctx, b, s)
+                       : p.lds == 32 ? launch_batch_kernel<BLOCK, 32, true, kLayoutW4>(ctx, b, s)
+                                     : launch_batch_kernel<BLOCK, 24, true, kLayoutW4>(ctx, b, s);
+        if (rc != kNoSpill) return rc;
+        b->whole_stacks = true;
     }
-    if (p.lds == 8) return launch_batch_kernel<BLOCK, 8, true, kLayoutW4>(ctx, b, s);
-    if (p.lds == 16) return launch_batch_kernel<BLOCK, 16, true, kLayoutW4>(ctx, b, s);
-    if (p.lds == 32) return launch_batch_kernel<BLOCK, 32, true, kLayoutW4>(ctx, b, s);
-    return launch_batch_kernel<BLOCK, 24, true, kLayoutW4>(ctx, b, s);
+    if (need <= 24) return launch_batch_kernel<BLOCK, 24, false, kLayoutW4>(ctx, b, s);
+    if (need <= 36) return launch_batch_kernel<BLOCK, 36, false, kLayoutW4>(ctx, b, s);
+    if (need <= 48) return launch_batch_kernel<BLOCK, 48, false, kLayoutW4>(ctx, b, s);
+    if (need <= 64) return launch_batch_kernel<BLOCK, 64, false, kLayoutW4>(ctx, b, s);
+    return launch_batch_kernel<BLOCK, kMaxWideStack, false, kLayoutW4>(ctx, b, s);
 }
 
 // The whole launch sequence on `s` (also what the graph captures).
@@ -431,15 +444,15 @@ std::string cache_key(const rt_batch* b) {
     return k.str();
 }
 
-template <bool DEEP>
+template <int STACK, bool DEEP>
 int launch_dyn_t(rt_ctx* ctx, const BatchIo& bio, uint32_t* cursor, uint32_t total, uint32_t stack_need,
                  uint32_t refill, hipStream_t s) {
-    auto kern = k_trace_batch<256, kStackLds, DEEP, kLayoutW4>;
+    auto kern = k_trace_batch<256, STACK, DEEP, kLayoutW4>;
     int32_t* spill = nullptr;
     if (DEEP) {
-        const int rc = stack_spill(ctx, stack_need - kStackLds, s, &spill);
+        const int rc = stack_spill(ctx, stack_need - STACK, s, &spill);
         if (rc) return rc;
-        if (!spill) return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: no stack spill area");
+        if (!spill) return kNoSpill;
     }
     int per_cu = 0;
     RT_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, 0));
@@ -461,8 +474,13 @@ int launch_batch_dynamic(rt_ctx* ctx, const BatchIo& bio, uint32_t* cursor, uint
     if (!total) return RT_OK;
     if (refill < 1u || refill > 64u) refill = 32u;
     if (stack_need > kMaxWideStack) return set_error(ctx, RT_ERR_UNSUPPORTED, "batch: a 4-wide tree deeper than 31 levels");
-    return stack_need <= kStackLds ? launch_dyn_t<false>(ctx, bio, cursor, total, stack_need, refill, s)
-                                   : launch_dyn_t<true>(ctx, bio, cursor, total, stack_need, refill, s);
+    if (stack_need <= 24) return launch_dyn_t<24, false>(ctx, bio, cursor, total, stack_need, refill, s);
+    const int rc = launch_dyn_t<24, true>(ctx, bio, cursor, total, stack_need, refill, s);
+    if (rc != kNoSpill) return rc;
+    if (stack_need <= 36) return launch_dyn_t<36, false>(ctx, bio, cursor, total, stack_need, refill, s);
+    if (stack_need <= 48) return launch_dyn_t<48, false>(ctx, bio, cursor, total, stack_need, refill, s);
+    if (stack_need <= 64) return launch_dyn_t<64, false>(ctx, bio, cursor, total, stack_need, refill, s);
+    return launch_dyn_t<kMaxWideStack, false>(ctx, bio, cursor, total, stack_need, refill, s);
 }
 
 int launch_gather(rt_ctx* ctx, const BatchIo& bio, const HostSpan* d_spans, rt_ray* d_rays, uint32_t total,

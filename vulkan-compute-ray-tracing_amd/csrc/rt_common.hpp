@@ -415,8 +415,9 @@ struct TraceArgs {
 };
 int launch_trace_packed(rt_ctx* ctx, const TraceArgs& a, hipStream_t s);
 // The context's area for stack entries past those in LDS, `entries` deep for
-// every lane of a launch; made on first use, null while `s` is capturing and
-// there is none yet.
+// every lane of a launch; made on first use, null where there is none yet and
+// memory is short or `s` is capturing.  Callers then launch a variant with
+// whole stacks in LDS.
 int stack_spill(rt_ctx* ctx, uint32_t entries, hipStream_t s, int32_t** out);
 constexpr int kNoSpill = -1;               // a launch's status: it needs an area it cannot have
 // The next block of the context's ray-cursor ring (kCursorBlock words; the

@@ -183,8 +183,11 @@ int stack_spill(rt_ctx* ctx, uint32_t entries, hipStream_t s, int32_t** out) {
     if (!ctx->d_spill[k]) {
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         if (s && hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone) return RT_OK;
-        RT_HIP(ctx, hipMalloc((void**)&ctx->d_spill[k],
-                              sizeof(int32_t) * kDepth[k] * (size_t)ctx->num_cus * kMaxLanesPerCu));
+        const size_t bytes = sizeof(int32_t) * kDepth[k] * (size_t)ctx->num_cus * kMaxLanesPerCu;
+        if (hipMalloc((void**)&ctx->d_spill[k], bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            ctx->d_spill[k] = nullptr;
+        }
     }
     *out = ctx->d_spill[k];
     return RT_OK;
@@ -398,7 +401,7 @@ int launch_trace_packed(rt_ctx* ctx, const TraceArgs& a, hipStream_t s) {
                            : p.lds == 16 ? launch_w4<16, true>(ctx, a, s, stats)
                            : p.lds == 32 ? launch_w4<32, true>(ctx, a, s, stats)
                                          : launch_w4<kStackLds, true>(ctx, a, s, stats);
-            // (no spill area during a capture that comes before the area exists)
+            // (no spill area: memory is short, or a capture comes before it exists)
             if (rc != kNoSpill) return rc;
         }
         if (need <= kStackLds) return launch_w4<kStackLds, false>(ctx, a, s, stats);
