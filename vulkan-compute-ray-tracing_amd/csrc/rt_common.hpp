@@ -278,6 +278,9 @@ struct rt_ctx {
     static constexpr int kWorkspaces = 6;
     void* ws[kWorkspaces] = {};
     size_t ws_bytes[kWorkspaces] = {};
+    // held from a scene's packing to its copy out of the scratch: a server's
+    // additions may come from any thread, beside its context's own uploads
+    std::mutex upload_mu;
     int32_t* d_spill[3] = {};         // stack entries past LDS (stack_spill), each made on first use
     uint32_t* d_counters = nullptr;   // kRenderCounters words: a render's live rays per bounce
     uint32_t* d_cursors = nullptr;    // ring of persistent-kernel ray cursors

@@ -804,6 +804,7 @@ extern "C" int rt_scene_upload(rt_ctx* ctx, const rt_scene_desc* desc, rt_scene*
     if (!ctx) return RT_ERR_INVALID;
     if (!desc || !out) return set_error(ctx, RT_ERR_INVALID, "rt_scene_upload: null argument");
     *out = nullptr;
+    std::lock_guard<std::mutex> up(ctx->upload_mu);
     PreparedScene prep;
     int rc = scene_prepare(ctx, desc, prep);
     if (rc) return rc;

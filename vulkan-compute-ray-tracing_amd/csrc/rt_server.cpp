@@ -137,7 +137,6 @@ struct rt_server {
     std::vector<Slot> slots;
     std::thread worker;
     std::mutex mu;
-    std::mutex upload_mu;
     std::condition_variable work_cv, done_cv;
     std::deque<Request*> pending;
     std::unordered_map<uint64_t, Request*> waited;
@@ -488,8 +487,8 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
     if (!S || !desc || !scene_id) return RT_ERR_INVALID;
     // validated and packed first, in scratch, so the scene's device bytes are
     // known before any of them is allocated
-    // (one upload at a time: its scratch is the context's)
-    std::lock_guard<std::mutex> up(S->upload_mu);
+    // (one upload at a time: its scratch is the context's, whoever else uses it)
+    std::lock_guard<std::mutex> up(S->ctx->upload_mu);
     PreparedScene prep;
     {
         int rc = scene_prepare(S->ctx, desc, prep);
@@ -607,7 +606,7 @@ extern "C" int rt_server_scene_remove(rt_server* S, uint64_t id) {
         S->resident -= it->second.bytes;
         S->scenes.erase(it);
     }
-    std::lock_guard<std::mutex> up(S->upload_mu);
+    std::lock_guard<std::mutex> up(S->ctx->upload_mu);
     rt_scene_release(S->ctx, sc);
     return RT_OK;
 }

@@ -422,20 +422,34 @@ struct WideTree {
     const rt_triangle* raw_tris = nullptr;    // the caller's arrays, when packed on the device
     const rt_bvh_node* raw_nodes = nullptr;
     ~WideTree() { if (own && base) (void)hipFree(base); }
-    // false: no room
+    // false: no room.  (Leaves the context's error text alone: that belongs to
+    // the thread that uses the context, which a server's additions need not be.)
     bool allocate(rt_ctx* ctx, size_t bytes) {
-        if (bytes <= kUploadKept) {
-            if (ensure_workspace(ctx, kWsUpload, bytes) == RT_OK) {
-                base = (char*)ctx->ws[kWsUpload];
-                return true;
-            }
-        } else if (hipMalloc((void**)&base, bytes) == hipSuccess) {
-            own = true;
+        void*& kept = ctx->ws[kWsUpload];
+        size_t& kept_bytes = ctx->ws_bytes[kWsUpload];
+        own = bytes > kUploadKept;
+        if (!own && kept_bytes >= bytes) {
+            base = (char*)kept;
             return true;
         }
-        (void)hipGetLastError();
-        base = nullptr;
-        return false;
+        if (!own && kept) {
+            // (waits for the kernels that use it)
+            (void)hipFree(kept);
+            kept = nullptr;
+            kept_bytes = 0;
+        }
+        const size_t grown = own ? bytes : bytes + bytes / 8;
+        if (hipMalloc((void**)&base, grown) != hipSuccess) {
+            (void)hipGetLastError();
+            base = nullptr;
+            own = false;
+            return false;
+        }
+        if (!own) {
+            kept = base;
+            kept_bytes = grown;
+        }
+        return true;
     }
     void bind(const WideLayout& L, uint32_t leaves, uint32_t records) {
         n = leaves;
