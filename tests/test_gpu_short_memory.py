@@ -67,3 +67,29 @@ def test_queries_without_room_for_a_stack_area(rt):
     sc.release()
     ctx.close()
     other.close()
+
+
+def hits_of(rt, ctx, host, rays):
+    scene = ctx.upload(host)
+    out = rt.hits_from_device(ctx.closest_hit(scene, rays))
+    scene.release()
+    return out
+
+
+# 262,144 triangles: scratch of 103 MiB that the context keeps, a scene of 63;
+# 1,048,576: 350 MiB given back after the upload, a scene of 250
+@pytest.mark.parametrize("tris,left", [(262144, 112), (1048576, 460)])
+def test_upload_without_room_for_its_scratch_and_the_scene(rt, tris, left):
+    hs = rt.scene_clusters(tris, 12)
+    rays = rt.rays_to_device(rt.rays_box(5000, 9, 4.0))
+    other = rt.Context(0)
+    want = hits_of(rt, other, hs, rays)
+    other.close()
+    ctx = rt.Context(0)
+    print(f"case: upload of {tris} triangles with {left} MiB left", flush=True)
+    with memory_left(left):
+        scene = ctx.upload(hs)
+    got = rt.hits_from_device(ctx.closest_hit(scene, rays))
+    assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
+    scene.release()
+    ctx.close()

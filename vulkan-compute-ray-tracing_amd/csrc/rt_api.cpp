@@ -15,6 +15,7 @@ int set_error(rt_ctx* ctx, int code, const std::string& msg) {
 
 int hip_error(rt_ctx* ctx, hipError_t e, const char* what) {
     std::string m = std::string(what) + ": " + hipGetErrorString(e);
+    (void)hipGetLastError();      // reported: not the next call's error too
     return set_error(ctx, e == hipErrorOutOfMemory ? RT_ERR_NOMEM : RT_ERR_HIP, m);
 }
 

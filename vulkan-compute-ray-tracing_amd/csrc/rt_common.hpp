@@ -216,6 +216,11 @@ struct PreparedScene {
 // `plain`: on the host, without a tree of its own (needs no device memory).
 int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& out, bool plain = false);
 int scene_commit(rt_ctx* ctx, PreparedScene& prep, rt_scene** out);
+// scene_commit; where memory is short for it, the traversal tree and the
+// upload's scratch are given up first (prep is then what was committed).
+int scene_commit_within(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& prep, rt_scene** out);
+// Frees the scratch that the context keeps for uploads (no prepared scene may be using it).
+void upload_scratch_release(rt_ctx* ctx);
 // Validates and packs `d` on the device (rt_pack.hpp); *done stays false
 // where the host has to.
 int device_pack(rt_ctx* ctx, const rt_scene_desc& d, PreparedScene& P, bool* done);

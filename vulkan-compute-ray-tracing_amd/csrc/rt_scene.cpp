@@ -752,6 +752,21 @@ int scene_commit(rt_ctx* ctx, PreparedScene& P, rt_scene** out) {
     return RT_OK;
 }
 
+void upload_scratch_release(rt_ctx* ctx) {
+    if (ctx->ws[kWsUpload]) (void)hipFree(ctx->ws[kWsUpload]);      // (waits for the kernels that use it)
+    ctx->ws[kWsUpload] = nullptr;
+    ctx->ws_bytes[kWsUpload] = 0;
+}
+
+int scene_commit_within(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& P, rt_scene** out) {
+    int rc = scene_commit(ctx, P, out);
+    if (rc != RT_ERR_NOMEM || (!P.wide && !ctx->ws[kWsUpload])) return rc;
+    P = PreparedScene{};
+    upload_scratch_release(ctx);
+    rc = scene_prepare(ctx, desc, P, true);
+    return rc ? rc : scene_commit(ctx, P, out);
+}
+
 int scene_binary_records(rt_ctx* ctx, rt_scene* s, uint32_t layout) {
     if (!s->fast) return RT_OK;
     std::lock_guard<std::mutex> lk(s->lazy_mu);
@@ -808,7 +823,7 @@ extern "C" int rt_scene_upload(rt_ctx* ctx, const rt_scene_desc* desc, rt_scene*
     PreparedScene prep;
     int rc = scene_prepare(ctx, desc, prep);
     if (rc) return rc;
-    return scene_commit(ctx, prep, out);
+    return scene_commit_within(ctx, desc, prep, out);
 }
 
 extern "C" int rt_scene_check(const rt_scene_desc* desc, rt_scene_info* info, char* err, size_t errlen) {

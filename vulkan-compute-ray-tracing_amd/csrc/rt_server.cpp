@@ -562,8 +562,12 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
         evicted.clear();
     }
     rt_scene* sc = nullptr;
-    int rc = scene_commit(S->ctx, prep, &sc);
+    int rc = scene_commit_within(S->ctx, desc, prep, &sc);
     std::lock_guard<std::mutex> lk(S->mu);
+    if (!rc) {                                    // (committed without its tree)
+        S->resident -= bytes - prep.bytes;
+        bytes = prep.bytes;
+    }
     if (rc) {
         S->resident -= bytes;
         S->st.scenes_refused++;
