@@ -93,3 +93,24 @@ def test_upload_without_room_for_its_scratch_and_the_scene(rt, tris, left):
     assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
     scene.release()
     ctx.close()
+
+
+def test_server_frees_scratch_before_scenes(rt):
+    """Adding a scene of about 60 MiB with 200 left, half of which its scratch takes:
+    no idle scene need go."""
+    hosts = [rt.scene_clusters(20000, 1), rt.scene_clusters(262144, 2)]
+    ctx = rt.Context(0)
+    srv = rt.Server(ctx, slots=1, max_batch_rays=1 << 16, max_render_pixels=1 << 16)
+    first = srv.add_scene(hosts[0])
+    print("case: server addition with 200 MiB left", flush=True)
+    with memory_left(200):
+        second = srv.add_scene(hosts[1])
+        assert sorted(srv.scenes()) == sorted([first, second])
+        assert srv.stats().scenes_evicted == 0
+    rays = rt.rays_box(5000, 9, 4.0)
+    hits = np.zeros(5000, rt.HIT_DT)
+    assert srv.wait(srv.submit_query(second, rays, hits)) == rt.RT_OK
+    want = hits_of(rt, ctx, hosts[1], rt.rays_to_device(rays))
+    assert np.array_equal(hits.view(np.uint8), want.view(np.uint8))
+    srv.close()
+    ctx.close()

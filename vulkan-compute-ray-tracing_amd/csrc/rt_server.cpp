@@ -537,7 +537,11 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
     for (;;) {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || (uint64_t)free_b >= bytes + margin) break;
-        // the traversal tree and its scratch go before any resident scene
+        // the traversal tree and the uploads' scratch go before any resident scene
+        if (!prep.wide && S->ctx->ws[kWsUpload]) {
+            upload_scratch_release(S->ctx);
+            continue;
+        }
         if (prep.wide) {
             prep = PreparedScene{};
             const int rc = scene_prepare(S->ctx, desc, prep, true);
