@@ -450,10 +450,12 @@ int rt_server_create(rt_ctx* ctx, const rt_server_config* config, rt_server** ou
 int rt_server_destroy(rt_server* server);
 /* Makes a scene resident.  Admission comes before the scene's own device
  * memory: it is validated and packed first (in the upload's scratch, or on
- * the host), which fixes its device
- * bytes; least recently used idle scenes are then evicted (and freed) while
- * the budget, or the device's free memory, cannot hold it, and only then is
- * it uploaded -- resident bytes never exceed the budget, not even during a
+ * the host), which fixes its device bytes.  Where the budget, or the device's
+ * free memory, cannot hold it, traversal trees are given up -- the new scene's,
+ * then those of resident scenes, least recently used first, each once its
+ * running requests have ended (a copy of the records that stay is made for it) --
+ * then least recently used idle scenes are evicted (and freed), and only then
+ * is it uploaded: resident bytes never exceed the budget, not even during a
  * swap.  RT_ERR_NOMEM when it cannot fit. */
 int rt_server_scene_add(rt_server* server, const rt_scene_desc* desc, uint64_t* scene_id);
 int rt_server_scene_remove(rt_server* server, uint64_t scene_id);

@@ -219,6 +219,10 @@ int scene_commit(rt_ctx* ctx, PreparedScene& prep, rt_scene** out);
 // scene_commit; where memory is short for it, the traversal tree and the
 // upload's scratch are given up first (prep is then what was committed).
 int scene_commit_within(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& prep, rt_scene** out);
+// Gives up the traversal tree of a resident scene that no launch is using; it
+// is traversed by the caller's records from then on.  The bytes freed: 0 where
+// it has no tree, or there is no room to move what stays.
+uint64_t scene_drop_tree(rt_ctx* ctx, rt_scene* s);
 // Frees the scratch that the context keeps for uploads (no prepared scene may be using it).
 void upload_scratch_release(rt_ctx* ctx);
 // Validates and packs `d` on the device (rt_pack.hpp); *done stays false
@@ -250,7 +254,9 @@ struct rt_scene {
     // from root4 on, the device-built tree's (wide); without one root4 is the
     // caller's root.  Both trees' leaves name d_ptris slots.
     int32_t root4 = rtamd::kEmptyRoot;
-    bool wide = false;
+    bool wide = false;                // d_ptris lie in a device-built tree's order
+    uint32_t tree_records = 0;        // records from root4 on; 0 without that tree, or once it is given up
+    uint32_t leaf_slots = 0;          // triangles in d_ptris
     uint32_t stack4 = 0;              // stack entries either tree needs, plus one
     uint32_t given_stack4 = 0;        // the caller's records alone
     rtamd::PTri* d_ptris = nullptr;

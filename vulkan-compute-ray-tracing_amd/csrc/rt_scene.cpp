@@ -730,6 +730,8 @@ int scene_commit(rt_ctx* ctx, PreparedScene& P, rt_scene** out) {
     s->root_ref = fast ? packed.root : kEmptyRoot;
     s->frame = packed.frame;
     s->root4 = !fast ? kEmptyRoot : s->wide ? (int32_t)P.given_records : packed.root4;
+    s->tree_records = P.wide ? P.wide_records : 0;
+    s->leaf_slots = P.leaf_slots;
     s->stack4 = fast ? std::max(packed.stack4, P.wide_need) : 0;
     s->given_stack4 = fast ? packed.stack4 : 0;
     P.wide.reset();
@@ -756,6 +758,32 @@ void upload_scratch_release(rt_ctx* ctx) {
     if (ctx->ws[kWsUpload]) (void)hipFree(ctx->ws[kWsUpload]);      // (waits for the kernels that use it)
     ctx->ws[kWsUpload] = nullptr;
     ctx->ws_bytes[kWsUpload] = 0;
+}
+
+uint64_t scene_drop_tree(rt_ctx* ctx, rt_scene* s) {
+    if (!s->tree_records) return 0;
+    const size_t records = (size_t)s->root4, slots = s->leaf_slots;
+    rt_scene to;
+    uint64_t bytes = 0;
+    bool ok = hipSetDevice(ctx->device) == hipSuccess && alloc_records(ctx, &to, records, slots, bytes) == RT_OK &&
+              hipMemcpyAsync(to.d_w4nodes, s->d_w4nodes, sizeof(PNode4) * records, hipMemcpyDeviceToDevice, nullptr) == hipSuccess &&
+              hipMemcpyAsync(to.d_ptris, s->d_ptris, sizeof(PTri) * slots, hipMemcpyDeviceToDevice, nullptr) == hipSuccess &&
+              hipStreamSynchronize(nullptr) == hipSuccess;
+    // the old records, or what was allocated of the new
+    const rt_scene* gone = ok ? s : &to;
+    const uint64_t was = packed_record_bytes((uint64_t)records + s->tree_records, slots);
+    (void)hipGetLastError();
+    if (gone->tri_off == kSeparateArrays && gone->d_ptris) (void)hipFree(gone->d_ptris);
+    if (gone->d_w4nodes) (void)hipFree(gone->d_w4nodes);
+    if (!ok) return 0;
+    s->d_w4nodes = to.d_w4nodes;
+    s->d_ptris = to.d_ptris;
+    s->tri_off = to.tri_off;
+    s->root4 = 0;
+    s->tree_records = 0;
+    s->stack4 = s->given_stack4;
+    s->info.device_bytes -= was - bytes;
+    return was - bytes;
 }
 
 int scene_commit_within(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& P, rt_scene** out) {

@@ -34,6 +34,9 @@ struct SrvScene {
     uint64_t bytes = 0;
     uint64_t last_use = 0;
     uint32_t refs = 0;           // queued or running requests
+    uint32_t running = 0;        // requests taken by a slot
+    bool held = false;           // no request is to be taken: its tree is being given up
+    bool keeps_tree = false;     // it could not be
 };
 
 struct Request {
@@ -294,6 +297,7 @@ void finish_request(rt_server* S, Request* r, int status) {
     r->done = true;
     auto it = S->scenes.find(r->scene_id);
     if (it != S->scenes.end() && it->second.refs) it->second.refs--;
+    if (it != S->scenes.end() && r->running) it->second.running--;
     if (status == RT_OK) {
         S->st.completed++;
         S->lat_ms.push_back((float)std::chrono::duration<double, std::milli>(r->t1 - r->t0).count());
@@ -331,6 +335,7 @@ void retire_slot(rt_server* S, Slot& sl) {
 void worker_main(rt_server* S) {
     (void)hipSetDevice(S->ctx->device);
     std::unique_lock<std::mutex> lk(S->mu);
+    auto held = [&](const Request* r) { return S->scenes[r->scene_id].held; };
     for (;;) {
         bool busy = false;
         for (Slot& sl : S->slots) {
@@ -362,6 +367,10 @@ void worker_main(rt_server* S) {
         }
         for (Slot& sl : S->slots) {
             if (sl.busy || S->pending.empty()) continue;
+            if (held(S->pending.front())) {
+                busy = true;            // not for long: look again
+                break;
+            }
             sl.render = S->pending.front()->kind == 1;
             sl.rays = 0;
             if (sl.render || S->cfg.mode == RT_SERVE_FIFO) {
@@ -370,13 +379,17 @@ void worker_main(rt_server* S) {
                 S->pending.pop_front();
             } else {
                 while (!S->pending.empty() && S->pending.front()->kind == 0 && sl.reqs.size() < kMaxItems &&
+                       !held(S->pending.front()) &&
                        sl.rays + S->pending.front()->n <= S->cfg.max_batch_rays) {
                     sl.rays += S->pending.front()->n;
                     sl.reqs.push_back(S->pending.front());
                     S->pending.pop_front();
                 }
             }
-            for (Request* r : sl.reqs) r->running = true;
+            for (Request* r : sl.reqs) {
+                r->running = true;
+                S->scenes[r->scene_id].running++;
+            }
             sl.busy = true;
             S->st.launches++;
             lk.unlock();
@@ -510,17 +523,64 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
         S->scenes.erase(victim);
         S->st.scenes_evicted++;
     };
-    // admission under the budget: evict, then reserve the new scene's bytes
+    // the new scene packed again without its traversal tree
+    auto prepare_plain = [&]() -> int {
+        prep = PreparedScene{};
+        const int rc = scene_prepare(S->ctx, desc, prep, true);
+        bytes = rc ? 0 : prep.bytes;
+        return rc ? fail(S, rc, std::string("rt_server_scene_add: ") + rt_last_error(S->ctx)) : RT_OK;
+    };
+    // The least recently used scene that has a traversal tree gives it up: no
+    // request of it is launched meanwhile, and those running end first.  Called
+    // with the lock held.
+    auto drop_tree = [&](std::unique_lock<std::mutex>& lk) -> bool {
+        uint64_t id = 0, oldest = UINT64_MAX;
+        for (auto& kv : S->scenes)
+            if (kv.second.scene->tree_records && !kv.second.keeps_tree && kv.second.last_use < oldest) {
+                oldest = kv.second.last_use;
+                id = kv.first;
+            }
+        if (!id) return false;
+        S->scenes[id].held = true;
+        rt_scene* const sc = S->scenes[id].scene;
+        // (removing it meanwhile frees it after this upload)
+        S->done_cv.wait(lk, [&] { return !S->scenes.count(id) || S->scenes[id].running == 0; });
+        if (!S->scenes.count(id)) return true;
+        lk.unlock();
+        const uint64_t freed = scene_drop_tree(S->ctx, sc);
+        lk.lock();
+        auto it = S->scenes.find(id);
+        if (it == S->scenes.end()) return true;
+        it->second.held = false;
+        it->second.keeps_tree = freed == 0;
+        it->second.bytes -= freed;
+        S->resident -= freed;
+        S->work_cv.notify_all();
+        return true;
+    };
+    // Admission under the budget.  Traversal trees take what it has to spare:
+    // they go, the new scene's first, before any scene is refused or evicted
+    // that the caller's records alone leave room for.  Then evict, and reserve
+    // the new scene's bytes.
     std::vector<rt_scene*> evicted;
     bool admitted = false;
     {
-        std::lock_guard<std::mutex> lk(S->mu);
-        while (budget && S->resident + bytes > budget) {
+        std::unique_lock<std::mutex> lk(S->mu);
+        for (;;) {
+            admitted = !budget || S->resident + bytes <= budget;
+            if (admitted) break;
+            if (prep.wide) {
+                lk.unlock();
+                const int rc = prepare_plain();
+                if (rc) return rc;
+                lk.lock();
+                continue;
+            }
+            if (bytes <= budget && drop_tree(lk)) continue;
             const uint64_t v = pick_victim();
             if (!v) break;
             evict(v, evicted);
         }
-        admitted = !budget || S->resident + bytes <= budget;
         if (admitted) {
             S->resident += bytes;
             S->peak = std::max(S->peak, S->resident);
@@ -537,23 +597,25 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
     for (;;) {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || (uint64_t)free_b >= bytes + margin) break;
-        // the traversal tree and the uploads' scratch go before any resident scene
+        // traversal trees and the uploads' scratch go before any resident scene
         if (!prep.wide && S->ctx->ws[kWsUpload]) {
             upload_scratch_release(S->ctx);
             continue;
         }
         if (prep.wide) {
-            prep = PreparedScene{};
-            const int rc = scene_prepare(S->ctx, desc, prep, true);
+            const uint64_t before = bytes;
+            const int rc = prepare_plain();
             std::lock_guard<std::mutex> lk(S->mu);
-            S->resident -= bytes;
-            bytes = rc ? 0 : prep.bytes;
-            S->resident += bytes;
+            S->resident -= before - bytes;
             if (rc) {
                 S->st.scenes_refused++;
-                return fail(S, rc, std::string("rt_server_scene_add: ") + rt_last_error(S->ctx));
+                return rc;
             }
             continue;
+        }
+        {
+            std::unique_lock<std::mutex> lk(S->mu);
+            if (drop_tree(lk)) continue;
         }
         uint64_t v = 0;
         {
