@@ -780,13 +780,12 @@ __device__ __forceinline__ void trace_persistent(const TraceScene& sc, const Tra
                     if (LAYOUT == kLayoutQ16 || kW4) {
                         bo = f3{(r.o.x - q.ox) * q.rx, (r.o.y - q.oy) * q.ry, (r.o.z - q.oz) * q.rz};
                         inv = f3{inv.x * q.sx, inv.y * q.sy, inv.z * q.sz};
-                        // the origin in the frame in double: within 2^-31 quanta
-                        // of where the quantizer's divisions put it
+                        // the origin in the frame in double, as the quantizer placed the bounds
                         double bod[3] = {0.0, 0.0, 0.0};
                         if (kW4) {
-                            bod[0] = ((double)r.o.x - (double)q.ox) * q.dx;
-                            bod[1] = ((double)r.o.y - (double)q.oy) * q.dy;
-                            bod[2] = ((double)r.o.z - (double)q.oz) * q.dz;
+                            bod[0] = quotient((double)r.o.x - (double)q.ox, (double)q.sx, q.dx);
+                            bod[1] = quotient((double)r.o.y - (double)q.oy, (double)q.sy, q.dy);
+                            bod[2] = quotient((double)r.o.z - (double)q.oz, (double)q.sz, q.dz);
                         }
                         if (!(fmaxf(fmaxf(fabsf(bo.x), fabsf(bo.y)), fabsf(bo.z)) < kFarOrigin))
                             reach = frame_far(r, q, bo, bod, t_shift);
