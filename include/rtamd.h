@@ -18,7 +18,7 @@
  *     own stream).  A context is externally synchronised.
  *   - All device work on one context must be ordered on ONE stream: a
  *     context's workspaces (the sorted trace order, render path state,
- *     traversal stacks) are shared by its launches, and calls return before
+ *     traversal stacks past their first entries) are shared by its launches, and calls return before
  *     their kernels finish.  Two launches of one context on different
  *     streams may overlap on the device and overwrite each other's
  *     workspaces.  Work that must overlap uses one context per stream (the
@@ -441,9 +441,10 @@ typedef struct rt_server_stats {
 } rt_server_stats;
 
 typedef struct rt_server rt_server;
-/* Page-locked host memory for request buffers: rays, hits and targets in
- * such memory are copied by DMA straight to and from the device; pageable
- * buffers go through the slot's staging copy. */
+/* Page-locked host memory for request buffers: a batch's kernels read rays
+ * and write hits in such memory where it lies (buffers not 8-byte aligned, and
+ * render targets, are copied by DMA); pageable buffers go through the slot's
+ * staging copy. */
 int rt_host_alloc(size_t bytes, void** out);
 int rt_host_free(void* p);
 int rt_server_create(rt_ctx* ctx, const rt_server_config* config, rt_server** out);

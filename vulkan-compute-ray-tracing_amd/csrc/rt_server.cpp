@@ -272,8 +272,9 @@ int launch_slot(rt_server* S, Slot& sl) {
         const HostSpan* const d_spans = (const HostSpan*)(sl.d_tables + at.spans);
         int rc = launch_gather(sl.ctx, bio, d_spans, sl.d_rays, off, sl.d_cursor, st);
         if (rc) return rc;
-        // refill threshold as for a plain query: early refills when most rays
-        // trace a large scene (long traversals), late ones otherwise
+        // early refills when most rays trace a large scene (long traversals),
+        // late ones otherwise.  (A plain query's thresholds were swept again for
+        // the present loop, launch_packed_t; a batch's were not.)
         const uint32_t refill = 2ull * long_rays >= off ? 24u : 48u;
         rc = launch_batch_dynamic(sl.ctx, bio, sl.d_cursor, off, need, refill, st);
         if (rc) return rc;

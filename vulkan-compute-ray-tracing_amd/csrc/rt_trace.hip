@@ -193,8 +193,10 @@ int stack_spill(rt_ctx* ctx, uint32_t entries, hipStream_t s, int32_t** out) {
     return RT_OK;
 }
 
-// Ray cursors for persistent launches: a ring of counters so launches on
-// different streams never share one.  A launch zeroes its block with a fill
+// Ray cursors for persistent launches: a ring of counters, a block of its own
+// for each of many launches in a row.  (A context's launches belong on one
+// stream all the same: they share its workspaces, the spill areas above among
+// them.)  A launch zeroes its block with a fill
 // kernel on its own stream right before use, unless the caller had an
 // earlier kernel on that stream do it (TraceArgs::cursor_zeroed).
 uint32_t* next_cursor(rt_ctx* ctx) {
