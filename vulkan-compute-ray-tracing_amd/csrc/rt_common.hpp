@@ -221,6 +221,7 @@ struct PreparedScene {
     bool device_packed = false;
     uint32_t given_records = 0, leaf_slots = 0;      // the caller's 4-wide records and the triangle slots
     uint64_t bytes = 0;                 // device bytes scene_commit allocates
+    uint64_t tree_bytes = 0;            // of them, the traversal tree's
 };
 // `plain`: on the host, without a tree of its own (needs no device memory).
 int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& out, bool plain = false);
@@ -387,8 +388,11 @@ int ensure_workspace(rt_ctx* ctx, int slot, size_t bytes);
 //   81,920-triangle icosphere, 300,000 camera   110   113   118    94
 //     500,000 shell                             164   149   156
 //   1080p, 4 samples, 4M triangles, ms         21.0  16.6  16.0  17.8
-// and at least 4, 8 or 16 rays a wave cost 22.6, 25.0 and 29.8 us against
-// 17.3 on 256 rays: down to one a wave.
+// The rule goes by rays alone and is not the best column of every row: four
+// waves from 448 rays a SIMD up cost the icosphere's 500,000 shell rays 5%
+// against three, and 2,000,000 camera rays would gain 8% with five.  At least 4,
+// 8 or 16 rays a wave cost 22.6, 25.0 and 29.8 us against 17.3 on 256 rays:
+// down to one a wave.
 struct LaunchPlan { uint32_t blocks, per_wave; };
 RT_HOST_DEVICE inline LaunchPlan plan_launch(uint32_t n, uint32_t grid, uint32_t waves_per_block, uint32_t simds) {
     const uint32_t load = n / simds + (n % simds != 0u);           // rays a SIMD

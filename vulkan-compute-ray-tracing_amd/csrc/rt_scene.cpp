@@ -641,7 +641,9 @@ int scene_prepare(rt_ctx* ctx, const rt_scene_desc* desc, PreparedScene& P, bool
     if (P.sphere_tree) b += sizeof(SphereNode) * (uint64_t)P.snodes.size();
     if (P.fast) {
         b += sizeof(int32_t) * (uint64_t)P.leaf_slots;
-        b += packed_record_bytes((uint64_t)P.given_records + P.wide_records, P.leaf_slots);
+        const uint64_t bare = packed_record_bytes(P.given_records, P.leaf_slots);
+        P.tree_bytes = packed_record_bytes((uint64_t)P.given_records + P.wide_records, P.leaf_slots) - bare;
+        b += bare + P.tree_bytes;
         if (P.with_pnodes) b += sizeof(PNode) * (uint64_t)P.packed.nodes.size();
         if (P.with_qnodes) b += sizeof(PNodeQ) * (uint64_t)P.packed.qnodes.size();
     }

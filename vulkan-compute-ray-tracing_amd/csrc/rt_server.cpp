@@ -32,11 +32,11 @@ using namespace rtamd;
 struct SrvScene {
     rt_scene* scene = nullptr;
     uint64_t bytes = 0;
+    uint64_t tree = 0;           // of them, those of a traversal tree it could give up
     uint64_t last_use = 0;
     uint32_t refs = 0;           // queued or running requests
     uint32_t running = 0;        // requests taken by a slot
     bool held = false;           // no request is to be taken: its tree is being given up
-    bool keeps_tree = false;     // it could not be
 };
 
 struct Request {
@@ -537,7 +537,7 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
     auto drop_tree = [&](std::unique_lock<std::mutex>& lk) -> bool {
         uint64_t id = 0, oldest = UINT64_MAX;
         for (auto& kv : S->scenes)
-            if (kv.second.scene->tree_records && !kv.second.keeps_tree && kv.second.last_use < oldest) {
+            if (kv.second.tree && kv.second.last_use < oldest) {
                 oldest = kv.second.last_use;
                 id = kv.first;
             }
@@ -553,31 +553,34 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
         auto it = S->scenes.find(id);
         if (it == S->scenes.end()) return true;
         it->second.held = false;
-        it->second.keeps_tree = freed == 0;
         it->second.bytes -= freed;
+        it->second.tree = 0;               // (none freed: it keeps its tree, which counts as its own)
         S->resident -= freed;
         S->work_cv.notify_all();
         return true;
     };
-    // Admission under the budget.  Traversal trees take what it has to spare:
-    // they go, the new scene's first, before any scene is refused or evicted
-    // that the caller's records alone leave room for.  Then evict, and reserve
-    // the new scene's bytes.
+    // Admission under the budget.  Scenes are evicted, or the new one refused,
+    // as if there were no traversal trees; trees take what the budget spares
+    // then, and go least recently used first, the new scene's last.
     std::vector<rt_scene*> evicted;
     bool admitted = false;
     {
         std::unique_lock<std::mutex> lk(S->mu);
         for (;;) {
+            uint64_t bare = bytes - prep.tree_bytes;
+            for (auto& kv : S->scenes) bare += kv.second.bytes - kv.second.tree;
             admitted = !budget || S->resident + bytes <= budget;
             if (admitted) break;
-            if (prep.wide) {
-                lk.unlock();
-                const int rc = prepare_plain();
-                if (rc) return rc;
-                lk.lock();
-                continue;
+            if (bare <= budget) {
+                if (bare + prep.tree_bytes <= budget && drop_tree(lk)) continue;
+                if (prep.wide) {
+                    lk.unlock();
+                    const int rc = prepare_plain();
+                    if (rc) return rc;
+                    lk.lock();
+                    continue;
+                }
             }
-            if (bytes <= budget && drop_tree(lk)) continue;
             const uint64_t v = pick_victim();
             if (!v) break;
             evict(v, evicted);
@@ -642,7 +645,7 @@ extern "C" int rt_server_scene_add(rt_server* S, const rt_scene_desc* desc, uint
                     std::string("rt_server_scene_add: upload: ") + rt_last_error(S->ctx));
     }
     uint64_t id = S->next_scene++;
-    S->scenes[id] = SrvScene{sc, bytes, S->tick++, 0};
+    S->scenes[id] = SrvScene{sc, bytes, prep.tree_bytes, S->tick++};
     S->st.scenes_added++;
     *scene_id = id;
     return RT_OK;
