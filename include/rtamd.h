@@ -451,13 +451,15 @@ int rt_server_create(rt_ctx* ctx, const rt_server_config* config, rt_server** ou
 int rt_server_destroy(rt_server* server);
 /* Makes a scene resident.  Admission comes before the scene's own device
  * memory: it is validated and packed first (in the upload's scratch, or on
- * the host), which fixes its device bytes.  Where the budget, or the device's
- * free memory, cannot hold it, traversal trees are given up -- the new scene's,
- * then those of resident scenes, least recently used first, each once its
- * running requests have ended (a copy of the records that stay is made for it) --
- * then least recently used idle scenes are evicted (and freed), and only then
- * is it uploaded: resident bytes never exceed the budget, not even during a
- * swap.  RT_ERR_NOMEM when it cannot fit. */
+ * the host), which fixes its device bytes.  Least recently used idle scenes
+ * are evicted (and freed) while the budget cannot hold the scenes without their
+ * traversal trees; trees have what it spares then: those of resident scenes are
+ * given up, least recently used first, until the new scene fits, each once its
+ * scene's running requests have ended (the records that stay are copied for it),
+ * and the new scene's own where it would not fit even so.  Short of device
+ * memory, trees and kept scratch go before scenes.  Only then is it uploaded:
+ * resident bytes never exceed the budget, not even during a swap.
+ * RT_ERR_NOMEM when it cannot fit. */
 int rt_server_scene_add(rt_server* server, const rt_scene_desc* desc, uint64_t* scene_id);
 int rt_server_scene_remove(rt_server* server, uint64_t scene_id);
 /* Writes up to `cap` resident scene ids; *count receives the total. */

@@ -283,8 +283,8 @@ __device__ __forceinline__ float shfl_f(float x, uint32_t src) {
 // grid]), which few rays ever reach.  Without DEEP the host has checked that
 // the scenes need no more than STACK.
 //
-// Work sharing in the drain (4-wide layouts, whole stack in LDS, no
-// counters; in batched launches the helper also takes the donor's scene):
+// Work sharing in the drain (4-wide layouts, entries in LDS, no counters; in
+// batched launches the helper also takes the donor's scene):
 // once a wave's rays are used up, its idle lanes would wait for the
 // longest rays of the wave.  Instead each idle lane takes the bottom entry of
 // a busy lane's stack -- the subtree that lane would visit last -- and
