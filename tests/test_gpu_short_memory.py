@@ -31,7 +31,7 @@ def memory_left(mib):
 
 
 def test_queries_without_room_for_a_stack_area(rt):
-    """The smallest area takes 32 MiB."""
+    """The smallest area takes 32 MiB, the batch's 35."""
     hs = rt.scene_clusters(600000, 12)
     n = 1 << 20
     rays_host = rt.rays_box(n, 9, 4.0)
@@ -49,8 +49,8 @@ def test_queries_without_room_for_a_stack_area(rt):
     pin_rays[:] = rays_host[:1 << 18]
     # (the batch's tables, and a first area of few blocks; the larger one finds no room)
     batch = rt.Batch(ctx, [(scene, rays, bhits)], rt.batch_config(blocks_per_cu=1, use_graph=0))
-    print("case: plain, batched and served query of a new context with 8 MiB left", flush=True)
-    with memory_left(8):
+    print("case: plain, batched and served query of a new context with 24 MiB left", flush=True)
+    with memory_left(24):
         ctx.closest_hit(scene, rays, hits)
         torch.cuda.synchronize()
         batch.set_config(rt.batch_config(stack_lds=8))
